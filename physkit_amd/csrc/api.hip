@@ -2042,7 +2042,7 @@ pkg_status pkg_gjk_epa_batch(pkg_ctx *ctx, uint32_t n, const int32_t *kind_a, co
         hipStream_t st = ctx->st;
         dbuf<int32_t> ka, kb, dh;
         dbuf<double> pa, pb, dv, dout;
-        dbuf<uint32_t> ba, ea, bb, eb, ua, ub;
+        dbuf<uint32_t> ba, ea, bb, eb, ua, ub, words, ovf;
         dbuf<char> pool;
         {
             std::vector<uint32_t> tag_a(n, 0u), tag_b(n, 0u);
@@ -2072,6 +2072,8 @@ pkg_status pkg_gjk_epa_batch(pkg_ctx *ctx, uint32_t n, const int32_t *kind_a, co
         dout.reserve(10 * static_cast<size_t>(n));
         dh.reserve(n);
         pool.reserve(epa_big_bytes());
+        words.reserve(4);
+        ovf.reserve(n);
         shape_pair_dev sp;
         sp.kind_a = ka.p;
         sp.kind_b = kb.p;
@@ -2084,7 +2086,7 @@ pkg_status pkg_gjk_epa_batch(pkg_ctx *ctx, uint32_t n, const int32_t *kind_a, co
         sp.verts = dv.p;
         sp.uv_a = ua.p;
         sp.uv_b = ub.p;
-        launch_gjk_epa_batch(sp, n, dout.p, dh.p, pool.p, st);
+        launch_gjk_epa_batch_dev(sp, n, n_verts, dout.p, dh.p, words.p, ovf.p, pool.p, 1, st);
         hip_check(hipGetLastError(), "batch launch");
         std::vector<double> o = download(dout, 10 * static_cast<size_t>(n), st);
         std::vector<int32_t> h = download(dh, n, st);

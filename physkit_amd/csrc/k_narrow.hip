@@ -8,7 +8,7 @@
 //   3. manifold update (warm-start transfer, persistence, add/reduce, events), one
 //      thread per pair, reading the previous step's manifold by source index.
 #include "pk_access.hpp"
-#include "pk_gjk.hpp"
+#include "pk_narrow.hpp"
 
 #include <type_traits>
 
@@ -17,25 +17,7 @@ namespace pk
 namespace
 {
 constexpr int kBlock = 256;
-constexpr int kEpaBlock = 64;
 unsigned grid(size_t n, int b = kBlock) { return static_cast<unsigned>((n + b - 1) / b); }
-
-// UV: the shapes may include tagged UV spheres (a kernel built without it carries no
-// code for their fast support)
-template <bool UV> __device__ __forceinline__ gshape body_shape(const bodies_dev &b, const shapes_dev &s, uint32_t id)
-{
-    gshape g;
-    g.kind = 2;
-    g.a = ld3(b.pos, b.n, id);
-    g.b = mk(0.0, 0.0, 0.0);
-    g.q = ldq(b.quat, b.n, id);
-    uint32_t sh = b.shape[id];
-    g.v = s.verts + 3 * static_cast<size_t>(s.voff[sh]);
-    g.nv = s.off[sh + 1] - s.off[sh];
-    g.uv = UV ? s.uv[sh] : 0u;
-    g.paired = 1;
-    return g;
-}
 
 // GJK cull. Two bodies are apart when their bounding spheres (radius: the largest
 // vertex distance from the shape origin) or their oriented local boxes (the shape's
@@ -199,44 +181,6 @@ __device__ __forceinline__ bool spheres32_apart(float4 a, float4 b)
     const float d = sqrtf(dx * dx + dy * dy + dz * dz);
     const float mag = ((fabsf(a.x) + fabsf(a.y)) + (fabsf(a.z) + fabsf(b.x))) + (fabsf(b.y) + fabsf(b.z));
     return d * (1.0f - 1e-5f) - 4e-7f * mag > (a.w + b.w) * (1.0f + 1e-5f) + 2e-6f;
-}
-
-// GJK simplex hand-off, planar: slot 0 = point count, then per point p.xyz and the
-// two support features packed in one 64-bit word (kSimplexWords doubles per hit).
-__device__ __forceinline__ void st_spt(double *d, uint32_t cap, uint32_t slot, int k, const spt &p)
-{
-    double *b = d + static_cast<size_t>(1 + 4 * k) * cap + slot;
-    b[0] = p.p.x;
-    b[cap] = p.p.y;
-    b[2 * static_cast<size_t>(cap)] = p.p.z;
-    b[3 * static_cast<size_t>(cap)] =
-        __longlong_as_double(static_cast<long long>((static_cast<uint64_t>(p.ib) << 32) | p.ia));
-}
-__device__ __forceinline__ spt ld_spt(const double *d, uint32_t cap, uint32_t slot, int k)
-{
-    const double *b = d + static_cast<size_t>(1 + 4 * k) * cap + slot;
-    spt p;
-    p.p = mk(b[0], b[cap], b[2 * static_cast<size_t>(cap)]);
-    uint64_t f = static_cast<uint64_t>(__double_as_longlong(b[3 * static_cast<size_t>(cap)]));
-    p.ia = static_cast<uint32_t>(f);
-    p.ib = static_cast<uint32_t>(f >> 32);
-    return p;
-}
-__device__ __forceinline__ void save_simplex(double *d, uint32_t cap, uint32_t slot, const simplex &x)
-{
-    d[slot] = static_cast<double>(x.n);
-    st_spt(d, cap, slot, 0, x.s0);
-    if (x.n > 1) st_spt(d, cap, slot, 1, x.s1);
-    if (x.n > 2) st_spt(d, cap, slot, 2, x.s2);
-    if (x.n > 3) st_spt(d, cap, slot, 3, x.s3);
-}
-__device__ __forceinline__ void load_simplex(const double *d, uint32_t cap, uint32_t slot, simplex &x)
-{
-    x.n = static_cast<int>(d[slot]);
-    x.s0 = ld_spt(d, cap, slot, 0);
-    if (x.n > 1) x.s1 = ld_spt(d, cap, slot, 1);
-    if (x.n > 2) x.s2 = ld_spt(d, cap, slot, 2);
-    if (x.n > 3) x.s3 = ld_spt(d, cap, slot, 3);
 }
 
 // A lane takes Q consecutive pairs; the pairs whose bodies are not apart (above) are
@@ -417,11 +361,6 @@ __global__ void __launch_bounds__(kBlock, 3) // 3 waves per SIMD fit without spi
         }
         __syncthreads(); // the next round's append reuses the same LDS
     }
-}
-
-__device__ __forceinline__ void write_info(double *info, uint32_t cap, uint32_t p, const double *o)
-{
-    for (int k = 0; k < 10; ++k) info[static_cast<size_t>(k) * cap + p] = o[k];
 }
 
 // one thread per hit, 192-face store in private memory; a solve that needs more is
@@ -765,40 +704,6 @@ __global__ void __launch_bounds__(kBlock)
 }
 
 // ---- standalone batch ----
-__device__ gshape pair_shape(const int32_t *kind, const double *prm, const uint32_t *vb, const uint32_t *ve,
-                             const double *verts, const uint32_t *uv, uint32_t i)
-{
-    const double *q = prm + 10 * static_cast<size_t>(i);
-    gshape g;
-    g.kind = kind[i];
-    g.v = nullptr;
-    g.nv = 0;
-    g.uv = 0;
-    g.paired = 0;
-    g.b = mk(0.0, 0.0, 0.0);
-    g.q = mkq(1.0, 0.0, 0.0, 0.0);
-    if (g.kind == 0)
-    {
-        g.a = mk(q[0], q[1], q[2]);
-        g.b = mk(q[3], q[4], q[5]);
-    }
-    else if (g.kind == 1)
-    {
-        g.a = mk(q[0], q[1], q[2]);
-        g.q = mkq(q[3], q[4], q[5], q[6]);
-        g.b = mk(q[7], q[8], q[9]);
-    }
-    else
-    {
-        g.a = mk(q[0], q[1], q[2]);
-        g.q = mkq(q[3], q[4], q[5], q[6]);
-        g.v = verts + 3 * static_cast<size_t>(vb[i]);
-        g.nv = ve[i] - vb[i];
-        g.uv = uv ? uv[i] : 0u; // no tags: every support scans all vertices (same results)
-    }
-    return g;
-}
-
 template <class S>
 __device__ void batch_one(const shape_pair_dev &sp, uint32_t i, double *out, int32_t *hit, S &store)
 {
@@ -817,53 +722,14 @@ __device__ void batch_one(const shape_pair_dev &sp, uint32_t i, double *out, int
     hit[i] = r == 1 ? 1 : (r == 0 ? 2 : 3);
 }
 
-__global__ void __launch_bounds__(kEpaBlock) k_batch(shape_pair_dev sp, uint32_t n, double *out, int32_t *hit)
-{
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    epa_store_fast store;
-    batch_one(sp, i, out, hit, store);
-}
-
-__global__ void k_batch_big(shape_pair_dev sp, uint32_t n, double *out, int32_t *hit,
-                            epa_store_big *pool)
-{
-    uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= 1) return;
-    // single thread walks the overflowed pairs one by one through the large store
-    for (uint32_t i = 0; i < n; ++i)
-        if (hit[i] == 3) batch_one(sp, i, out, hit, pool[0]);
-}
-// ---- standalone batch over device arrays with caller-free scratch ----
 // Scratch words: [0] pairs with invalid input, [1] pairs listed for the large store,
 // [2] pairs that overflowed the large store as well.
 __global__ void k_batch_dev_clear(uint32_t *words)
 {
     if (threadIdx.x < 4) words[threadIdx.x] = 0u;
 }
-__global__ void __launch_bounds__(kEpaBlock)
-    k_batch_dev(shape_pair_dev sp, uint32_t n, uint32_t n_verts, double *out, int32_t *hit, uint32_t *words,
-                uint32_t *ovf_list)
-{
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    // the host variant checks these on the host (pkg_gjk_epa_batch)
-    for (int side = 0; side < 2; ++side)
-    {
-        const int k = side ? sp.kind_b[i] : sp.kind_a[i];
-        const uint32_t vb = side ? sp.vbeg_b[i] : sp.vbeg_a[i], ve = side ? sp.vend_b[i] : sp.vend_a[i];
-        if (k < 0 || k > 2 || (k == 2 && (ve <= vb || ve > n_verts)))
-        {
-            hit[i] = -1;
-            atomicAdd(&words[0], 1u);
-            return;
-        }
-    }
-    epa_store_fast store;
-    batch_one(sp, i, out, hit, store);
-    if (hit[i] == 3) ovf_list[atomicAdd(&words[1], 1u)] = i;
-}
-// one thread per large store, each taking every n_stores-th listed pair
+// one thread per large store, each taking every n_stores-th listed pair (solves past the
+// wavefront kernel's 512 faces, or with a plane distance that is not finite)
 __global__ void k_batch_dev_big(shape_pair_dev sp, double *out, int32_t *hit, uint32_t *words,
                                 const uint32_t *ovf_list, epa_store_big *stores, uint32_t n_stores)
 {
@@ -887,7 +753,7 @@ void launch_gjk_epa_batch_dev(const shape_pair_dev &sp, uint32_t n, uint32_t n_v
 {
     k_batch_dev_clear<<<1, 64, 0, st>>>(words);
     if (!n) return;
-    k_batch_dev<<<grid(n, kEpaBlock), kEpaBlock, 0, st>>>(sp, n, n_verts, out, hit, words, ovf_list);
+    launch_batch_wave(sp, n, n_verts, out, hit, words, ovf_list, st);
     k_batch_dev_big<<<1, 64, 0, st>>>(sp, out, hit, words, ovf_list, static_cast<epa_store_big *>(stores), n_stores);
 }
 
@@ -1001,14 +867,6 @@ bool cull_uses_records(uint32_t n_pairs, uint32_t n_bodies)
     // per-body records pay off with several pairs per body (hull clusters: 4; the
     // batched worlds, 0.6, read the planar arrays faster)
     return static_cast<size_t>(n_pairs) >= 2 * static_cast<size_t>(n_bodies);
-}
-
-void launch_gjk_epa_batch(const shape_pair_dev &sp, uint32_t n, double *out, int32_t *hit,
-                          void *big_pool, hipStream_t st)
-{
-    if (!n) return;
-    k_batch<<<grid(n, kEpaBlock), kEpaBlock, 0, st>>>(sp, n, out, hit);
-    if (big_pool) k_batch_big<<<1, 64, 0, st>>>(sp, n, out, hit, static_cast<epa_store_big *>(big_pool));
 }
 
 } // namespace pk

@@ -419,9 +419,8 @@ template <int G, bool UV = true> __device__ __forceinline__ bool gjk(const gshap
     return false;
 }
 
-// collision.cpp:191-248
-template <int G, bool UV = true>
-__device__ __forceinline__ bool pad_simplex(const gshape &A, const gshape &B, simplex &x, int gl)
+// collision.cpp:191-248; support(d) is the Minkowski support search
+template <class Support> __device__ __forceinline__ bool pad_simplex_with(simplex &x, Support &&support)
 {
     // stage k fills slot k (1: s1 from direction +x, 2: s2 off the line s0-s1, 3: s3
     // off the plane), each retried once in the opposite direction; written as one
@@ -444,7 +443,7 @@ __device__ __forceinline__ bool pad_simplex(const gshape &A, const gshape &B, si
 #pragma nounroll
         for (int att = 0; att < 2; ++att)
         {
-            p = msupport<G, UV>(A, B, att == 0 ? dir : -dir, gl);
+            p = support(att == 0 ? dir : -dir);
             if (att == 1) break;
             bool again;
             if (k == 1)
@@ -466,7 +465,11 @@ __device__ __forceinline__ bool pad_simplex(const gshape &A, const gshape &B, si
     double triple = dot(ad, cross(bd, cd));
     return fabs(triple) > 1e-12;
 }
-
+template <int G, bool UV = true>
+__device__ __forceinline__ bool pad_simplex(const gshape &A, const gshape &B, simplex &x, int gl)
+{
+    return pad_simplex_with(x, [&](v3 d) { return msupport<G, UV>(A, B, d, gl); });
+}
 
 // ---------------- EPA (collision.cpp:251-509) ----------------
 // One thread per solve. The polytope lives in a store of compile-time capacity

@@ -335,9 +335,10 @@ struct shape_pair_dev
     const double *verts;
     const uint32_t *uv_a, *uv_b; // UV-sphere tags of mesh shapes (0: none)
 };
-void launch_gjk_epa_batch(const shape_pair_dev &sp, uint32_t n, double *out, int32_t *hit,
-                          void *big_pool, hipStream_t st);
-// The same over device arrays with scratch the caller does not allocate: words (4 x u32:
+// one wavefront per pair; overflows of its store are listed (words[1]) in ovf_list
+void launch_batch_wave(const shape_pair_dev &sp, uint32_t n, uint32_t n_verts, double *out, int32_t *hit, uint32_t *words,
+                       uint32_t *ovf_list, hipStream_t st);
+// The batch over device arrays: words (4 x u32:
 // invalid pairs, pairs listed for the large store, pairs that overflowed it too; cleared
 // by the first launch), ovf_list (n entries) and n_stores large EPA stores. Invalid pairs
 // get hit = -1. uv tags may be null.

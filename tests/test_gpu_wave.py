@@ -1,0 +1,70 @@
+"""The wavefront-per-pair narrowphase against the oracle, bit for bit, where its layout has
+edges: vertex counts around the 32 lanes that search one shape (one vertex per lane up to
+32, strides above), equal supports and equal plane distances (axis-aligned boxes on a
+grid: heap ties), polytopes past the first stores' faces, and values that are not finite."""
+import numpy as np
+import pytest
+
+from test_gpu_parity import _assert_same, _oracle_shape
+
+pytestmark = pytest.mark.gpu
+
+
+def _hull(rng, n):
+    v = rng.normal(size=(n, 3))
+    return v / np.linalg.norm(v, axis=1, keepdims=True) * rng.uniform(0.3, 0.6, 3)
+
+
+def _quat(rng):
+    q = rng.normal(size=4)
+    return q / np.linalg.norm(q)
+
+
+def _cases(oracle, rng, what):
+    if isinstance(what, int):  # meshes of `what` vertices against meshes of 1-70
+        return [((2, np.concatenate([rng.normal(size=3) * 0.1, _quat(rng)]), _hull(rng, what)),
+                 (2, np.concatenate([rng.normal(size=3) * 0.25, _quat(rng)]), _hull(rng, int(rng.integers(1, 71)))))
+                for _ in range(96)]
+    box = oracle.box_verts((0.5, 0.5, 0.5))
+    out = []
+    if what == "grid":
+        for d in np.ndindex(4, 4, 4):
+            c = np.array(d) * 0.25
+            out.append(((2, [0, 0, 0, 1, 0, 0, 0], box), (2, np.concatenate([c, [1, 0, 0, 0]]), box)))
+            out.append(((0, [-0.5, -0.5, -0.5, 0.5, 0.5, 0.5], None), (1, np.concatenate([c, [1, 0, 0, 0], [0.5, 0.5, 0.5]]), None)))
+    elif what == "faces":  # dense spheres without the generator's vertex order: full scans, long solves
+        sph = oracle.sphere_verts(0.5, 16, 32)[::-1].copy()
+        for _ in range(24):
+            u = rng.normal(size=3)
+            out.append(((2, np.concatenate([[0, 0, 0], _quat(rng)]), sph),
+                        (2, np.concatenate([u / np.linalg.norm(u) * rng.uniform(0.0, 0.6), _quat(rng)]), sph)))
+    else:
+        for bad in (np.nan, np.inf, 1e200, 1e308):
+            for k in range(3):
+                p = np.zeros(3)
+                p[k] = bad
+                out.append(((2, np.concatenate([p, [1, 0, 0, 0]]), box), (2, [0.1, 0, 0, 1, 0, 0, 0], box)))
+                v = box.copy()
+                v[k, k] = bad
+                out.append(((2, [0, 0, 0, 1, 0, 0, 0], v), (2, [0.1, 0.2, 0, 1, 0, 0, 0], box)))
+    return out
+
+
+@pytest.mark.parametrize("what", [1, 2, 5, 31, 32, 33, 64, 65, "grid", "faces", "not finite"])
+def test_batch_edges_bitexact(pk, oracle, what):
+    rng = np.random.default_rng(4711)
+    cases = _cases(oracle, rng, what)
+    print(f"[wave] {what}: {len(cases)} pairs", flush=True)
+    g = pk.GpuWorld()
+    hit, out = g.gjk_epa_batch([c[0] for c in cases], [c[1] for c in cases])
+    g.close()
+    for i, (a, b) in enumerate(cases):
+        with np.errstate(all="ignore"):
+            r = oracle.gjk_epa(_oracle_shape(oracle, a), _oracle_shape(oracle, b))
+        if r is None:
+            assert hit[i] == 0, i
+        elif r == "degenerate":
+            assert hit[i] == 2, i
+        else:
+            assert hit[i] == 1, i
+            _assert_same(i, "gjk_epa", out[i], np.concatenate([r["normal"], r["world_a"], r["world_b"], [r["depth"]]]))
