@@ -304,15 +304,16 @@ typedef struct pkg_tuning
                               candidates, else 4 */
     int32_t epa_block;     /* threads per workgroup of the one-solve-per-thread EPA kernel: 64, 128
                               or 256 (default 64) */
-    uint32_t epa_lds_max;  /* GJK-hit batches of at most this many run one EPA solve per workgroup
-                              with the polytope in LDS; larger ones one solve per thread (512) */
+    uint32_t epa_lds_max;  /* GJK-hit batches of at most this many run one EPA solve per wavefront,
+                              the faces in its registers and points and heap in LDS; larger ones
+                              one solve per thread (default 2^32 - 1: every batch) */
     uint32_t tree_refits;  /* steps between full LBVH builds that refit the last build's hierarchy
                               to the new leaf boxes instead (0-64; default 7; 0 builds every
                               step). Pairs and query answers do not depend on the tree's shape,
                               so this changes only the walks' cost. Not chosen by pkg_autotune */
     float gjk_ms[4];       /* pkg_autotune: GJK stage ms per step with 1, 2, 4, 8 lanes per pair */
     float epa_block_ms[3]; /* EPA stage ms per step with workgroups of 64, 128, 256 threads */
-    float epa_lds_ms[3];   /* EPA stage ms per step with epa_lds_max 0, 512, 4096 */
+    float epa_lds_ms[3];   /* EPA stage ms per step with epa_lds_max 0, 4096, 2^32 - 1 */
 } pkg_tuning;
 
 /* Picks the launch shapes above by timing them on this world. It takes `steps` real

@@ -766,7 +766,13 @@ void pkg_ctx::step_once(double dt, hipEvent_t *ev, bool defer_pos)
         g.info = info.p;
         g.cap = static_cast<uint32_t>(std::min({hit_list.cap, ovf_list.cap, simplex.cap / kSimplexWords, info.cap / 10}));
     };
-    size_hits(std::min<uint32_t>(Pn, last_hits + last_hits / 2));
+    // One wavefront per pair runs GJK and EPA in one kernel, each list entry its own hit
+    // entry, when few pairs are expected (as the last step's; launch_gjk tells why);
+    // launch shapes that were set or tuned keep the separate stages.
+    const uint64_t expect = last.steps_total ? last.gjk_fp64 + last.gjk_fp64 / 4 : Pn;
+    const bool fused = !trials && !tuned && expect <= kWavePairs;
+    const uint32_t want_hits = fused ? static_cast<uint32_t>(expect) : last_hits + last_hits / 2;
+    size_hits(std::min<uint32_t>(Pn, want_hits));
     if (Pn)
     {
         gjk_list.reserve(Pn);
@@ -791,8 +797,9 @@ void pkg_ctx::step_once(double dt, hipEvent_t *ev, bool defer_pos)
         auto gjk_stage = [&](int group, bool again)
         {
             if (again)
-                for (int c : {C_GJK_LIST, C_GJK_LIST2, C_HITS, C_MLIVE}) reset_counter(c);
-            launch_gjk(keys[nxt].p, Pn, b, s, has_uv, group, g, gjk_list.p, cull_rec.p, f32, mo, counters.p, st);
+                for (int c : {C_GJK_LIST, C_GJK_LIST2, C_HITS, C_MLIVE, C_EPA_OVF}) reset_counter(c);
+            const gjk_wave_in wv{fused, static_cast<uint32_t>(expect), ovf_list.p};
+            launch_gjk(keys[nxt].p, Pn, b, s, has_uv, group, g, gjk_list.p, cull_rec.p, f32, wv, mo, counters.p, st);
         };
         gjk_stage(tune.gjk_group, false);
         record(ev, 4, st);
@@ -800,47 +807,45 @@ void pkg_ctx::step_once(double dt, hipEvent_t *ev, bool defer_pos)
         uint32_t hits = static_cast<uint32_t>(h_counters[C_HITS]);
         if (h_counters[C_MLIVE] > live_cap)
             throw pk_error(PKG_DEVICE_ERROR, "more culled pairs with contacts than manifolds with contacts");
-        if (hits > g.cap)
+        // the entries the hit lists need: the hits, or with the fused kernel the listed pairs
+        auto entries = [&]
+        { return static_cast<uint32_t>(h_counters[!fused ? C_HITS : (f32.s32 ? C_GJK_LIST2 : C_GJK_LIST)]); };
+        if (const uint32_t need = entries(); need > g.cap)
         {
-            // more hits than the hit lists hold: grow them and run the stage again
-            size_hits(hits + hits / 4);
+            // more than the hit lists hold: grow them and run the stage again
+            size_hits(need + need / 4);
             gjk_stage(tune.gjk_group, true);
             record(ev, 4, st);
             read_counters(C_HITS, C_MLIVE);
             hits = static_cast<uint32_t>(h_counters[C_HITS]);
-            if (hits > g.cap) throw pk_error(PKG_DEVICE_ERROR, "GJK hit count changed between identical runs");
+            if (entries() > g.cap) throw pk_error(PKG_DEVICE_ERROR, "GJK hit count changed between identical runs");
         }
         last_hits = hits;
-        // the EPA stage, with overflow reruns in larger stores (capacity never changes a
-        // result); it writes every hit's status and contact, so it too can run again
+        // overflowed solves rerun in larger stores (capacity never changes a result)
+        auto epa_reruns = [&](uint32_t novf)
+        {
+            if (!novf) return;
+            ovf2_list.reserve(novf);
+            launch_epa_wave(keys[nxt].p, ovf_list.p, novf, b, s, has_uv, true, g, ovf2_list.p, counters.p + C_EPA_OVF2, st);
+            const uint32_t n2 = static_cast<uint32_t>(read_counter(C_EPA_OVF2));
+            if (!n2) return;
+            big_pool.reserve(static_cast<size_t>(n2) * epa_big_bytes());
+            launch_epa_big(keys[nxt].p, ovf2_list.p, n2, b, s, g, big_pool.p, counters.p, st);
+            if (read_counter(C_EPA_BIG_FAIL)) throw pk_error(PKG_OVERFLOW_EPA, "EPA polytope exceeded 4096 faces");
+        };
+        // the EPA stage writes every hit's status and contact, so it too can run again
         auto epa_stage = [&](const tuning &tu, bool again)
         {
             if (again)
                 for (int c : {C_EPA_OVF, C_EPA_OVF2, C_EPA_BIG_FAIL}) reset_counter(c);
             launch_epa(keys[nxt].p, hits, b, s, has_uv, tu, g, ovf_list.p, counters.p, st);
-            const uint32_t novf = static_cast<uint32_t>(read_counter(C_EPA_OVF));
-            if (!novf) return;
-            // a small batch already ran with the LDS store: its overflows go straight to
-            // the global-memory store
-            const uint32_t *big_in = ovf_list.p;
-            uint32_t n2 = novf;
-            if (!epa_first_tier_is_lds(hits, tu))
-            {
-                ovf2_list.reserve(novf);
-                launch_epa_lds(keys[nxt].p, ovf_list.p, novf, b, s, g, ovf2_list.p, counters.p, st);
-                n2 = static_cast<uint32_t>(read_counter(C_EPA_OVF2));
-                big_in = ovf2_list.p;
-            }
-            if (n2)
-            {
-                big_pool.reserve(static_cast<size_t>(n2) * epa_big_bytes());
-                launch_epa_big(keys[nxt].p, big_in, n2, b, s, g, big_pool.p, counters.p, st);
-                if (read_counter(C_EPA_BIG_FAIL))
-                    throw pk_error(PKG_OVERFLOW_EPA, "EPA polytope exceeded 4096 faces");
-            }
+            if (hits) epa_reruns(static_cast<uint32_t>(read_counter(C_EPA_OVF)));
         };
         record(ev, 9, st);
-        epa_stage(tune, false);
+        if (fused)
+            epa_reruns(static_cast<uint32_t>(h_counters[C_EPA_OVF]));
+        else
+            epa_stage(tune, false);
         record(ev, 5, st);
         if (trials)
         {
@@ -855,7 +860,7 @@ void pkg_ctx::step_once(double dt, hipEvent_t *ev, bool defer_pos)
                 return static_cast<double>(ms);
             };
             static const int lanes[4] = {1, 2, 4, 8}, blocks[3] = {64, 128, 256};
-            static const uint32_t lds_max[3] = {0u, 512u, 4096u};
+            static const uint32_t lds_max[3] = {0u, 4096u, 0xFFFFFFFFu};
             for (int c = 0; c < 4; ++c) trials->gjk[c] += timed([&] { gjk_stage(lanes[c], true); });
             if (read_counter(C_HITS) != hits) throw pk_error(PKG_DEVICE_ERROR, "GJK hit count changed between runs");
             tuning tu = tune;
@@ -1863,7 +1868,7 @@ pkg_status pkg_autotune(pkg_ctx *ctx, double dt, int steps, pkg_tuning *out)
                 return b;
             };
             static const int lanes[4] = {1, 2, 4, 8}, blocks[3] = {64, 128, 256};
-            static const uint32_t lds_max[3] = {0u, 512u, 4096u};
+            static const uint32_t lds_max[3] = {0u, 4096u, 0xFFFFFFFFu};
             tuning &tu = ctx->tune;
             tu.gjk_group = lanes[argmin(tr.gjk, 4)];
             tu.epa_block = blocks[argmin(tr.epa_block, 3)];

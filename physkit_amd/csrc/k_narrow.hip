@@ -2,9 +2,10 @@
 // 244-320) split into three passes so each runs dense:
 //   1. GJK, one thread per active pair; hits are compacted (wavefront-aggregated
 //      append) with their final simplex;
-//   2. EPA, one thread per hit, polytope/faces/heap in a private 192-face store;
-//      a hit that needs more faces is rerun by a second kernel with a 4096-face store
-//      in global memory, so capacity never changes a result;
+//   2. EPA, one wavefront per hit (k_wave.hip), or one thread per hit with the polytope in a
+//      private 192-face store (pkg_tuning.epa_lds_max); a hit that needs more faces is rerun
+//      with 512, then with a 4096-face store in global memory, so capacity never changes a
+//      result. Short pair lists run passes 1 and 2 in one kernel, a wavefront per pair;
 //   3. manifold update (warm-start transfer, persistence, add/reduce, events), one
 //      thread per pair, reading the previous step's manifold by source index.
 #include "pk_access.hpp"
@@ -364,7 +365,7 @@ __global__ void __launch_bounds__(kBlock, 3) // 3 waves per SIMD fit without spi
 }
 
 // one thread per hit, 192-face store in private memory; a solve that needs more is
-// listed for the 4096-face kernel below
+// listed for the reruns
 template <bool UV, int BS>
 __global__ void __launch_bounds__(BS)
     k_epa(const uint64_t *keys, uint32_t n_hits, bodies_dev b, shapes_dev s, gjk_out_dev g,
@@ -389,35 +390,6 @@ __global__ void __launch_bounds__(BS)
     }
     unsigned long long slot = wave_append(&counters[C_EPA_OVF], ovf);
     if (ovf) ovf_list[slot] = h;
-}
-
-// Second tier: one workgroup per hit that overflowed the private store, its polytope in
-// LDS (896 faces): LDS round trips instead of global-memory ones on the solve's long
-// chain of dependent accesses. A solve that needs more goes on to k_epa_big.
-template <class S, bool UV>
-__global__ void __launch_bounds__(64)
-    k_epa_lds(const uint64_t *keys, const uint32_t *ovf_list, uint32_t n_ovf, bodies_dev b, shapes_dev s,
-              gjk_out_dev g, uint32_t *ovf2_list, unsigned long long *counters, int out_slot)
-{
-    __shared__ S store;
-    const uint32_t t = blockIdx.x;
-    if (t >= n_ovf || threadIdx.x != 0) return;
-    const uint32_t h = ovf_list ? ovf_list[t] : t;
-    const uint32_t p = g.hit_list[h];
-    const uint64_t key = keys[p];
-    gshape A = body_shape<UV>(b, s, static_cast<uint32_t>(key >> 32));
-    gshape B = body_shape<UV>(b, s, static_cast<uint32_t>(key & 0xFFFFFFFFu));
-    simplex x;
-    load_simplex(g.simplex, g.cap, h, x);
-    double out[10];
-    const int r = epa_solve<UV>(A, B, x, store, out);
-    if (r == 3)
-    {
-        ovf2_list[atomicAdd(&counters[out_slot], 1ull)] = h;
-        return;
-    }
-    if (r == 1) write_info(g.info, g.cap, h, out);
-    g.status[p] = static_cast<uint8_t>(r == 1 ? 1 : 2);
 }
 
 template <bool UV>
@@ -746,7 +718,6 @@ __global__ void k_batch_dev_big(shape_pair_dev sp, double *out, int32_t *hit, ui
 } // namespace
 
 size_t epa_big_bytes() { return sizeof(epa_store_big); }
-bool epa_first_tier_is_lds(uint32_t n_hits, const tuning &tu) { return n_hits <= tu.epa_lds_max; }
 
 void launch_gjk_epa_batch_dev(const shape_pair_dev &sp, uint32_t n, uint32_t n_verts, double *out, int32_t *hit,
                               uint32_t *words, uint32_t *ovf_list, void *stores, uint32_t n_stores, hipStream_t st)
@@ -758,8 +729,8 @@ void launch_gjk_epa_batch_dev(const shape_pair_dev &sp, uint32_t n, uint32_t n_v
 }
 
 void launch_gjk(const uint64_t *keys, uint32_t n_pairs, const bodies_dev &b, const shapes_dev &s, bool uv, int group,
-                gjk_out_dev &g, uint32_t *list, double *cull_rec, const gjk32_in &f32, const cull_manifold_out &mo,
-                unsigned long long *counters, hipStream_t st)
+                gjk_out_dev &g, uint32_t *list, double *cull_rec, const gjk32_in &f32, const gjk_wave_in &wv,
+                const cull_manifold_out &mo, unsigned long long *counters, hipStream_t st)
 {
     if (!n_pairs) return;
     if (cull_uses_records(n_pairs, b.n))
@@ -779,6 +750,11 @@ void launch_gjk(const uint64_t *keys, uint32_t n_pairs, const bodies_dev &b, con
         launch_gjk32(keys, list, n_pairs, b, *f32.s32, uv, f32.src, f32.prev_count, g.status, f32.list2, counters, st);
         list = f32.list2;
         slot = C_GJK_LIST2;
+    }
+    if (wv.on)
+    {
+        launch_gjk_epa_wave(keys, list, slot, wv.expect, b, s, uv, g, wv.ovf_list, counters, st);
+        return;
     }
     // sized for every pair up to kListGrid workgroups, which then step through the list
     // (its count is read on the device); groups past the listed count exit at once
@@ -804,14 +780,9 @@ void launch_epa(const uint64_t *keys, uint32_t n_hits, const bodies_dev &b, cons
                 const tuning &tu, gjk_out_dev &g, uint32_t *ovf_list, unsigned long long *counters, hipStream_t st)
 {
     if (!n_hits) return;
-    if (epa_first_tier_is_lds(n_hits, tu))
+    if (n_hits <= tu.epa_lds_max)
     {
-        if (uv)
-            k_epa_lds<epa_store_lds, true><<<n_hits, 64, 0, st>>>(keys, nullptr, n_hits, b, s, g, ovf_list, counters,
-                                                                 C_EPA_OVF);
-        else
-            k_epa_lds<epa_store_lds, false><<<n_hits, 64, 0, st>>>(keys, nullptr, n_hits, b, s, g, ovf_list,
-                                                                  counters, C_EPA_OVF);
+        launch_epa_wave(keys, nullptr, n_hits, b, s, uv, false, g, ovf_list, &counters[C_EPA_OVF], st);
         return;
     }
     auto go = [&](auto block)
@@ -828,15 +799,6 @@ void launch_epa(const uint64_t *keys, uint32_t n_hits, const bodies_dev &b, cons
     case 256: go(std::integral_constant<int, 256>{}); break;
     default: go(std::integral_constant<int, 64>{}); break;
     }
-}
-
-void launch_epa_lds(const uint64_t *keys, const uint32_t *ovf_list, uint32_t n_ovf, const bodies_dev &b,
-                    const shapes_dev &s, const gjk_out_dev &g, uint32_t *ovf2_list, unsigned long long *counters,
-                    hipStream_t st)
-{
-    if (n_ovf)
-        k_epa_lds<epa_store_lds, true><<<n_ovf, 64, 0, st>>>(keys, ovf_list, n_ovf, b, s, g, ovf2_list, counters,
-                                                            C_EPA_OVF2);
 }
 
 void launch_epa_big(const uint64_t *keys, const uint32_t *ovf_list, uint32_t n_ovf,

@@ -1,5 +1,6 @@
-// The standalone narrowphase (pkg_gjk_epa_batch, pkg_gjk_epa_batch_device) with a wavefront
-// per pair (pk_wave.hpp).
+// Narrowphase kernels that give each pair a wavefront (pk_wave.hpp): the step's GJK and
+// EPA for pair lists too short to fill the chip one thread per pair, EPA reruns, and the
+// standalone batch. Results are those of the one-thread kernels in k_narrow.hip.
 #include "pk_narrow.hpp"
 #include "pk_wave.hpp"
 
@@ -8,8 +9,95 @@ namespace pk
 namespace
 {
 constexpr int kWave = 64;
-constexpr int kBatchSlots = 8; // faces per lane: 512, enough for nearly every 64-expansion solve
+// faces a wavefront holds per lane: 3 (192 faces) for a step's solves, as the one-thread
+// kernel's first store; 8 (512) for reruns and for the batch, whose meshes are the caller's
+constexpr int kStepSlots = 3, kBatchSlots = 8;
 
+// the shape of this lane's side of pair `key`
+template <bool UV>
+__device__ __forceinline__ wave::shape pair_side(const bodies_dev &b, const shapes_dev &s, uint64_t key)
+{
+    const uint32_t id = wave::upper() ? static_cast<uint32_t>(key & 0xFFFFFFFFu) : static_cast<uint32_t>(key >> 32);
+    return wave::make_shape(body_shape<UV>(b, s, id));
+}
+
+// the contact or the status of hit h (pair p); an overflow is listed with its simplex
+template <bool UV, int K>
+__device__ __forceinline__ void solve_hit(const wave::shape &w, simplex &x, wave::store<K> &st, uint32_t p, uint32_t h,
+                                          const gjk_out_dev &g, uint32_t *ovf_list, unsigned long long *ovf_count)
+{
+    double out[10];
+    const int r = wave::epa_solve<UV, true, K>(w, x, st, out);
+    if (__lane_id() == 0)
+    {
+        if (r == 1) write_info(g.info, g.cap, h, out);
+        g.status[p] = static_cast<uint8_t>(r == 1 ? 1 : (r == 0 ? 2 : 3));
+        if (r == 3)
+        {
+            save_simplex(g.simplex, g.cap, h, x);
+            ovf_list[atomicAdd(ovf_count, 1ull)] = h;
+        }
+    }
+}
+
+// GJK and EPA of the listed pairs, one wavefront each: bounded by the longest pair's chain
+// (about 1.9 us per EPA expansion, 64 at most; 20 us on one thread with its store in private
+// memory), not by throughput. kWavePairs tells which lists take it. Entry i of the list is hit i if it
+// hits: its contact goes to entry i of the hit arrays (entries past g.cap are counted only;
+// the host sees the list's count, grows the arrays and runs the stage again), so no slot is
+// reserved per hit; each wavefront adds its hits to the counter once.
+template <bool UV>
+__global__ void __launch_bounds__(kWave)
+    k_gjk_epa_wave(const uint64_t *keys, const uint32_t *list, int list_slot, bodies_dev b, shapes_dev s, gjk_out_dev g,
+                   uint32_t *ovf_list, unsigned long long *counters)
+{
+    __shared__ wave::store<kStepSlots> st;
+    const uint32_t n_list = static_cast<uint32_t>(counters[list_slot]);
+    uint32_t hits = 0;
+    for (uint32_t i = blockIdx.x; i < n_list; i += gridDim.x)
+    {
+        const uint32_t p = wave::first32(list[i]);
+        const wave::shape w = pair_side<UV>(b, s, keys[p]);
+        simplex x;
+        const bool hit = wave::gjk<UV, true>(w, x);
+        if (hit) ++hits;
+        if (hit && i < g.cap)
+        {
+            if (__lane_id() == 0)
+            {
+                g.hit_list[i] = p;
+                g.hit_of[p] = i;
+            }
+            solve_hit<UV, kStepSlots>(w, x, st, p, i, g, ovf_list, &counters[C_EPA_OVF]);
+        }
+        else if (__lane_id() == 0)
+            g.status[p] = 0;
+    }
+    if (__lane_id() == 0 && hits) atomicAdd(&counters[C_HITS], static_cast<unsigned long long>(hits));
+}
+
+// EPA of hits in_list[0..n) (0..n-1 when null), one wavefront each: 0.12 ms on 535 hits of
+// UV spheres, boxes and hulls (one thread each 0.45 ms), 0.15 on 8,000 hull hits (0.45), 0.51
+// on 35,000 mixed hits (1.09), 0.18 on 17,880 box hits (0.36) and 2.08 on 143,000 hull hits
+// (2.07).
+template <bool UV, int K>
+__global__ void __launch_bounds__(kWave)
+    k_epa_wave(const uint64_t *keys, const uint32_t *in_list, uint32_t n, bodies_dev b, shapes_dev s, gjk_out_dev g,
+               uint32_t *ovf_list, unsigned long long *ovf_count)
+{
+    __shared__ wave::store<K> st;
+    if (blockIdx.x >= n) return;
+    const uint32_t h = in_list ? wave::first32(in_list[blockIdx.x]) : blockIdx.x;
+    const uint32_t p = wave::first32(g.hit_list[h]);
+    const wave::shape w = pair_side<UV>(b, s, keys[p]);
+    simplex x;
+    x.s1 = x.s2 = x.s3 = spt{mk(0.0, 0.0, 0.0), 0u, 0u};
+    load_simplex(g.simplex, g.cap, h, x);
+    x.n = static_cast<int>(wave::first32(static_cast<uint32_t>(x.n)));
+    solve_hit<UV, K>(w, x, st, p, h, g, ovf_list, ovf_count);
+}
+
+// ---- standalone batch ----
 // words as k_batch_dev_big (k_narrow.hip) reads them. The kernel is bound by the issue of its
 // dependent FP64 chains. One thread per pair took 7.9 ms on 65,536 pairs of boxes, hulls and
 // 482-vertex spheres (each lane scanning 2 x 482 vertices per support, the wavefront waiting
@@ -53,6 +141,37 @@ __global__ void __launch_bounds__(kWave)
     if (r == 3) ovf_list[atomicAdd(&words[1], 1u)] = i;
 }
 } // namespace
+
+void launch_gjk_epa_wave(const uint64_t *keys, const uint32_t *list, int list_slot, uint32_t expect, const bodies_dev &b,
+                         const shapes_dev &s, bool uv, const gjk_out_dev &g, uint32_t *ovf_list,
+                         unsigned long long *counters, hipStream_t st)
+{
+    // one wavefront per expected pair up to what the chip holds, then several pairs each
+    const uint32_t gr = std::min<uint32_t>(std::max<uint32_t>(expect, 256u), 8192u);
+    if (uv)
+        k_gjk_epa_wave<true><<<gr, kWave, 0, st>>>(keys, list, list_slot, b, s, g, ovf_list, counters);
+    else
+        k_gjk_epa_wave<false><<<gr, kWave, 0, st>>>(keys, list, list_slot, b, s, g, ovf_list, counters);
+}
+
+void launch_epa_wave(const uint64_t *keys, const uint32_t *in_list, uint32_t n, const bodies_dev &b, const shapes_dev &s,
+                     bool uv, bool rerun, const gjk_out_dev &g, uint32_t *ovf_list, unsigned long long *ovf_count,
+                     hipStream_t st)
+{
+    if (!n) return;
+    auto go = [&](auto slots)
+    {
+        constexpr int K = decltype(slots)::value;
+        if (uv)
+            k_epa_wave<true, K><<<n, kWave, 0, st>>>(keys, in_list, n, b, s, g, ovf_list, ovf_count);
+        else
+            k_epa_wave<false, K><<<n, kWave, 0, st>>>(keys, in_list, n, b, s, g, ovf_list, ovf_count);
+    };
+    if (rerun)
+        go(std::integral_constant<int, kBatchSlots>{});
+    else
+        go(std::integral_constant<int, kStepSlots>{});
+}
 
 void launch_batch_wave(const shape_pair_dev &sp, uint32_t n, uint32_t n_verts, double *out, int32_t *hit, uint32_t *words,
                        uint32_t *ovf_list, hipStream_t st)

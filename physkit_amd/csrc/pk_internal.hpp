@@ -88,7 +88,7 @@ enum counter_slot
     C_EPA_BIG_FAIL = 9,
     C_EVENTS = 10,
     C_TREE_FAIL = 11,
-    C_EPA_OVF2 = 12, // overflows of the LDS store, rerun in global memory
+    C_EPA_OVF2 = 12, // overflows of the 512-face store, rerun in global memory
     C_KEEP = 13,
     C_ISL_MAX = 14,
     C_NCOL = 15,
@@ -271,6 +271,24 @@ struct gjk32_in
     const uint8_t *prev_count;
     uint32_t *list2;
 };
+// GJK and EPA of every listed pair by a wavefront each (k_wave.hip): entry i of the list is
+// entry i of the hit arrays, and the stage ends with each hit's contact. expect: the pairs
+// expected (sizes the grid; the kernel reads the count).
+// Longer lists take the separate stages: k_gjk's 32-64 pairs per wavefront then fill the
+// chip and spend less on each (GJK and EPA in ms, separate / fused: 535 sphere, box and hull
+// pairs of 1,934 listed 0.34 / 0.13; 752 of 755 box pairs 0.11 / 0.07; 2,092 of 2,301
+// 0.70 / 0.48; 17,879 of 17,886 box pairs 0.23 / 0.29; 56,165 of 84,521 1.09 / 1.17;
+// 143,064 of 361,508 hull pairs 2.9 / 4.3).
+constexpr uint32_t kWavePairs = 8192;
+struct gjk_wave_in
+{
+    bool on;
+    uint32_t expect;
+    uint32_t *ovf_list;
+};
+void launch_gjk_epa_wave(const uint64_t *keys, const uint32_t *list, int list_slot, uint32_t expect, const bodies_dev &b,
+                         const shapes_dev &s, bool uv, const gjk_out_dev &g, uint32_t *ovf_list,
+                         unsigned long long *counters, hipStream_t st);
 // What the cull also settles of the manifold update: a pair whose bodies are apart has
 // no new contact, so its next manifold is empty unless it had contacts (prev_count of
 // its source, source_of(src, p), above 0). The cull writes every pair's next count,
@@ -287,28 +305,25 @@ struct cull_manifold_out
     uint32_t live_cap;
 };
 void launch_gjk(const uint64_t *keys, uint32_t n_pairs, const bodies_dev &b, const shapes_dev &s, bool uv, int group,
-                gjk_out_dev &g, uint32_t *list, double *cull_rec, const gjk32_in &f32, const cull_manifold_out &mo,
-                unsigned long long *counters, hipStream_t st);
+                gjk_out_dev &g, uint32_t *list, double *cull_rec, const gjk32_in &f32, const gjk_wave_in &wv,
+                const cull_manifold_out &mo, unsigned long long *counters, hipStream_t st);
 // Launch shapes the autotuner picks (pkg_autotune); none changes a result.
 struct tuning
 {
     int gjk_group = 4;           // lanes per pair in k_gjk (1, 2, 4, 8): 64 / gjk_group pairs per wavefront
     int epa_block = 64;          // threads per workgroup of k_epa (64, 128, 256)
-    uint32_t epa_lds_max = 512;  // batches of at most this many GJK hits run one EPA solve per workgroup
-                                 // with the LDS store (k_epa_lds); larger ones one per thread
+    uint32_t epa_lds_max = 0xFFFFFFFFu; // batches of at most this many GJK hits run one EPA solve per
+                                        // wavefront (k_epa_wave); larger ones one per thread (k_epa)
     uint32_t tree_refits = 7;    // steps that refit the last LBVH hierarchy between full builds
 };
 void launch_epa(const uint64_t *keys, uint32_t n_hits, const bodies_dev &b, const shapes_dev &s, bool uv,
                 const tuning &tu, gjk_out_dev &g, uint32_t *ovf_list, unsigned long long *counters, hipStream_t st);
-// overflowed hits rerun with an LDS store; its own overflows are listed in ovf2_list
-// (count at counters[C_EPA_OVF2]) for launch_epa_big
-void launch_epa_lds(const uint64_t *keys, const uint32_t *ovf_list, uint32_t n_ovf, const bodies_dev &b,
-                    const shapes_dev &s, const gjk_out_dev &g, uint32_t *ovf2_list, unsigned long long *counters,
-                    hipStream_t st);
+// EPA of hits in_list[0..n) (0..n-1 when null), one wavefront each: 192 faces, or 512 for a
+// rerun of overflows; its own overflows are listed in ovf_list (count at *ovf_count)
+void launch_epa_wave(const uint64_t *keys, const uint32_t *in_list, uint32_t n, const bodies_dev &b, const shapes_dev &s,
+                     bool uv, bool rerun, const gjk_out_dev &g, uint32_t *ovf_list, unsigned long long *ovf_count,
+                     hipStream_t st);
 size_t epa_big_bytes();
-// launch_epa runs batches this small with the LDS store already (its overflows skip
-// launch_epa_lds)
-bool epa_first_tier_is_lds(uint32_t n_hits, const tuning &tu);
 void launch_epa_big(const uint64_t *keys, const uint32_t *ovf_list, uint32_t n_ovf,
                     const bodies_dev &b, const shapes_dev &s, gjk_out_dev &g, void *pool,
                     unsigned long long *counters, hipStream_t st);
