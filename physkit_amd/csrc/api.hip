@@ -243,7 +243,7 @@ struct pkg_ctx
 
     // solver
     dbuf<uint32_t> colour, colour_start, order, order_alt;
-    dbuf<uint32_t> par, iv, iv_alt, iflags, ipos, istarts; // contact islands
+    dbuf<uint32_t> par, icnt, ibase, iroot, irank, iv, iv_alt, iflags, ipos, istarts; // contact islands
     dbuf<uint64_t> ik, ik_alt;
     dbuf<uint64_t> ckeys, ckeys_alt;
     dbuf<double> rows_s;      // solver rows in solve order
@@ -917,6 +917,7 @@ void pkg_ctx::step_once(double dt, hipEvent_t *ev, bool defer_pos)
     // ---- 4. contacts and joints (constraint.h:1052-1201)
     n_colours = 0;
     n_listed = 0;
+    bool chunked = false; // solved by k_solve_chunks
     const uint32_t n_joints = static_cast<uint32_t>(jkey_h.size());
     if (solve && (Pn || n_joints))
     {
@@ -928,27 +929,65 @@ void pkg_ctx::step_once(double dt, hipEvent_t *ev, bool defer_pos)
         // for the FP32 solve.
         auto write_rows = [&](const uint32_t *ord, uint32_t n_act, const rows_dev &rs, uint32_t scap)
         { launch_contact_setup(keys[nxt].p, n_act, ord, scap, b, MF(nxt), rs, dt, thr, f32, st); };
+        bool solved = false;
+        uint32_t longest = 0; // manifolds of the longest contact island (all-ones: not known)
         if (Pn)
         {
             colour.reserve(ncap);
-            claim.reserve(std::max<uint32_t>(n, 1));
             clist.reserve(std::max<uint32_t>(mdcap[nxt], 1));
-            // The manifolds with rows are listed as they are flagged (C_NLIST, from zero at
-            // the step's start), and the colouring rounds read that count on the device
-            // over a grid sized by the list's capacity: the row count, the list count and
-            // the colouring's state come back together at its first check.
-            launch_row_flags(keys[nxt].p, Pn, b, MF(nxt), colour.p, clist.p, counters.p, st);
             const uint32_t lcap = static_cast<uint32_t>(std::min<size_t>(clist.cap, 0xFFFFFFFFu));
+            // The manifolds with rows are listed as they are flagged (C_NLIST, from zero at
+            // the step's start) and, without joints, their bodies united into islands.
+            const bool islands = n_joints == 0;
+            if (islands)
             {
-                const unsigned long long *nl_dev = counters.p + C_NLIST;
-                const uint32_t *wo = nullptr, *pb = nullptr;
-                if (n_worlds > 1)
+                par.reserve(std::max<uint32_t>(n, 1));
+                icnt.reserve(std::max<uint32_t>(n, 1));
+                launch_island_init(par.p, icnt.p, n, st);
+            }
+            launch_row_flags(keys[nxt].p, Pn, b, MF(nxt), colour.p, clist.p, islands ? par.p : nullptr, counters.p, st);
+            const uint32_t *wo = nullptr, *pb = nullptr;
+            if (n_worlds > 1)
+            {
+                pair_base.reserve(n_worlds);
+                launch_pair_base(keys[nxt].p, Pn, world_of.p, pair_base.p, st);
+                wo = world_of.p;
+                pb = pair_base.p;
+            }
+            if (islands)
+            {
+                iroot.reserve(lcap);
+                irank.reserve(lcap);
+                launch_island_roots(keys[nxt].p, clist.p, lcap, b, par.p, icnt.p, iroot.p, irank.p, counters.p, st);
+                read_counters(C_ISL_CUR, C_NLIST); // rows, the list count and the longest island in one wait
+                nl = static_cast<uint32_t>(h_counters[C_NLIST]);
+                longest = static_cast<uint32_t>(std::min<unsigned long long>(h_counters[C_ISL_MAX], 0xFFFFFFFFull));
+                if (nl && longest <= static_cast<uint32_t>(f32 ? kChunkMax32 : kChunkMax))
                 {
-                    pair_base.reserve(n_worlds);
-                    launch_pair_base(keys[nxt].p, Pn, world_of.p, pair_base.p, st);
-                    wo = world_of.p;
-                    pb = pair_base.p;
+                    const uint32_t *ord = clist.p, *isl = nullptr;
+                    if (nl > static_cast<uint32_t>(kChunkTwoLanes))
+                    {
+                        ibase.reserve(std::max<uint32_t>(n, 1));
+                        iv.reserve(nl);
+                        iv_alt.reserve(nl);
+                        launch_island_group(clist.p, nl, icnt.p, n, iroot.p, irank.p, ibase.p, iv.p, iv_alt.p, counters.p,
+                                            st);
+                        ord = iv.p;
+                        isl = iv_alt.p;
+                    }
+                    record(ev, 10, st);
+                    launch_solve_chunks(keys[nxt].p, ord, isl, nl, longest, b, MF(nxt), colour.p, wo, pb,
+                                        cfg.solver_iterations, dt, thr, f32, counters.p, st);
+                    record(ev, 11, st);
+                    solved = chunked = true;
                 }
+            }
+            if (!solved && (nl || !islands))
+            {
+                // Global colouring: the rounds read the list's count on the device over a grid
+                // sized by the list's capacity.
+                const unsigned long long *nl_dev = counters.p + C_NLIST;
+                claim.reserve(std::max<uint32_t>(n, 1));
                 used.reserve(std::max<uint32_t>(n, 1));
                 launch_fill_u64(used.p, 0ull, n, st);
                 launch_fill_u64(claim.p, 0ull, n, st);
@@ -984,17 +1023,17 @@ void pkg_ctx::step_once(double dt, hipEvent_t *ev, bool defer_pos)
                     nl = static_cast<uint32_t>(h_counters[C_NLIST]);
                     c = static_cast<uint32_t>(h_counters[C_NCOL]);
                 }
+                else
+                    nl = 0;
             }
         }
         n_colours = c;
         n_listed = nl;
         if (n_joints) joint_prepare(b, dt);
-        bool solved = false;
-        if (c && !n_joints && c <= kIslandMaxColours)
+        if (!solved && c && !n_joints && c <= kIslandMaxColours && longest <= kIslandMaxManifolds)
         {
-            // one workgroup per chunk of whole contact islands when every island is small enough
-            // over the listed row manifolds only
-            par.reserve(std::max<uint32_t>(n, 1));
+            // long islands: one workgroup per chunk of whole islands, rows in memory, over
+            // the listed row manifolds sorted by (island, colour)
             ik.reserve(nl);
             ik_alt.reserve(nl);
             iv.reserve(nl);
@@ -1003,18 +1042,14 @@ void pkg_ctx::step_once(double dt, hipEvent_t *ev, bool defer_pos)
             ipos.reserve(nl);
             istarts.reserve(nl);
             bsums.reserve(scan_block_sums(nl));
-            total.reserve(2);
-            reset_counter(C_ISL_MAX);
-            island_sort is = launch_island_sort(keys[nxt].p, colour.p, clist.p, nl, c, b, par.p, ik.p, iv.p,
-                                                ik_alt.p, iv_alt.p, counters.p + C_ISL_MAX, sc, st);
-            launch_island_segments(is, nl, iflags.p, ipos.p, bsums.p, total.p, istarts.p, total.p + 1, st);
-            // island count, row manifold count and the longest island in one wait
-            launch_island_maxlen(istarts.p, total.p, nl, counters.p + C_ISL_MAX, st);
-            uint32_t h2[2] = {0, 0};
-            hip_check(hipMemcpyAsync(h2, total.p, 2 * sizeof(uint32_t), hipMemcpyDeviceToHost, st), "island count");
-            read_counters(C_ISL_MAX, C_ISL_MAX);
-            const uint32_t n_isl = h2[0], n_act = h2[1];
-            if (h_counters[C_ISL_MAX] <= kIslandMaxManifolds)
+            total.reserve(1);
+            island_sort is = launch_island_sort(keys[nxt].p, colour.p, clist.p, nl, c, n, iroot.p, ik.p, iv.p, ik_alt.p,
+                                                iv_alt.p, sc, st);
+            launch_island_segments(is, nl, iflags.p, ipos.p, bsums.p, total.p, istarts.p, st);
+            uint32_t n_isl = 0;
+            hip_check(hipMemcpyAsync(&n_isl, total.p, sizeof(uint32_t), hipMemcpyDeviceToHost, st), "island count");
+            hip_check(hipStreamSynchronize(st), "stream sync");
+            const uint32_t n_act = nl;
             {
                 const uint32_t scap = std::max<uint32_t>(n_act, 1);
                 rows_s.reserve(static_cast<size_t>(4) * scap * kRowF);
@@ -1025,8 +1060,8 @@ void pkg_ctx::step_once(double dt, hipEvent_t *ev, bool defer_pos)
                 rs.valid = row_valid_s.p;
                 write_rows(is.ord, n_act, rs, scap);
                 record(ev, 10, st);
-                launch_solve_islands(keys[nxt].p, is, istarts.p, n_isl, n_act, c, b, rs, scap,
-                                     cfg.solver_iterations, static_cast<uint32_t>(h_counters[C_ISL_MAX]), f32, st);
+                launch_solve_islands(keys[nxt].p, is, istarts.p, n_isl, n_act, c, b, rs, scap, cfg.solver_iterations, f32,
+                                     st);
                 record(ev, 11, st);
                 if (f32)
                     launch_impulse_writeback32(is.ord, n_act, MF(nxt), rs, scap, st);
@@ -1035,7 +1070,7 @@ void pkg_ctx::step_once(double dt, hipEvent_t *ev, bool defer_pos)
                 solved = true;
             }
         }
-        if (!solved)
+        if (!solved && (c || n_joints))
         {
             // per-colour launches: each pass sweeps the joint colours, then the manifold
             // colours (pass 0 warm starts, constraint.h:1123-1130; then the iterations)
@@ -1114,6 +1149,8 @@ void pkg_ctx::step_once(double dt, hipEvent_t *ev, bool defer_pos)
     last.gjk_hits = h_counters[C_HITS];
     last.contacts = h_counters[C_CONTACTS];
     last.rows = h_counters[C_ROWS];
+    // the island solve colours as it goes: its colour count comes with the step's counters
+    if (chunked) n_colours = static_cast<uint32_t>(h_counters[C_NCOL]);
     last.colours = n_colours;
     last.epa_overflow = h_counters[C_EPA_OVF];
     last.candidates = candidates;

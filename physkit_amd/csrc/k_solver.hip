@@ -7,9 +7,8 @@
 // Colouring: each round, every uncoloured manifold whose priority (mix32(p) << 32 | p)
 // is the minimum claim at each of its dynamic bodies takes the smallest colour free at
 // those bodies.
-#include "pk_access.hpp"
+#include "pk_solver.hpp"
 
-#include <cfloat>
 #include <type_traits>
 
 namespace pk
@@ -18,114 +17,6 @@ namespace
 {
 constexpr int kBlock = 256;
 unsigned grid(size_t n) { return static_cast<unsigned>((n + kBlock - 1) / kBlock); }
-
-struct rowv
-{
-    v3 Jv, Jwa, Jwb;
-    double Meff, bias, acc;
-};
-struct body_state
-{
-    v3 vel, ang;
-    double im;
-    m3 Iwi;
-    bool stat;
-};
-
-__device__ __forceinline__ double row_jv(const rowv &r, const body_state &A, const body_state &B)
-{ return ((dot(r.Jv, A.vel) + dot(r.Jwa, A.ang)) - dot(r.Jv, B.vel)) + dot(r.Jwb, B.ang); }
-
-__device__ __forceinline__ void row_apply(rowv &r, double lo, double hi, body_state &A, body_state &B) // :49-72
-{
-    double jv = row_jv(r, A, B);
-    double cfp = 0.0 * r.acc;
-    double lambda = -((jv + r.bias) + cfp) * r.Meff;
-    double old = r.acc;
-    double v = old + lambda;
-    r.acc = (v < lo) ? lo : ((hi < v) ? hi : v);
-    double ap = r.acc - old;
-    if (!A.stat)
-    {
-        A.vel = A.vel + (r.Jv * ap) * A.im;
-        A.ang = A.ang + mul(A.Iwi, r.Jwa * ap);
-    }
-    if (!B.stat)
-    {
-        B.vel = B.vel + ((-r.Jv) * ap) * B.im;
-        B.ang = B.ang + mul(B.Iwi, r.Jwb * ap);
-    }
-}
-
-__device__ __forceinline__ void row_warm(const rowv &r, body_state &A, body_state &B) // :74-87
-{
-    if (r.acc == 0.0) return;
-    if (!A.stat)
-    {
-        A.vel = A.vel + (r.Jv * r.acc) * A.im;
-        A.ang = A.ang + mul(A.Iwi, r.Jwa * r.acc);
-    }
-    if (!B.stat)
-    {
-        B.vel = B.vel + ((-r.Jv) * r.acc) * B.im;
-        B.ang = B.ang + mul(B.Iwi, r.Jwb * r.acc);
-    }
-}
-
-__device__ __forceinline__ void friction_block(rowv &t1, rowv &t2, double mu, double nacc, double i11,
-                                               double i12, double i22, body_state &A, body_state &B) // :1131-1187
-{
-    double maxf = mu * nacc;
-    double jv1 = row_jv(t1, A, B);
-    double jv2 = row_jv(t2, A, B);
-    double b1 = jv1 + 0.0;
-    double b2 = jv2 + 0.0;
-    double l1 = -(i11 * b1 + i12 * b2);
-    double l2 = -(i12 * b1 + i22 * b2);
-    double o1 = t1.acc, o2 = t2.acc;
-    double n1 = o1 + l1, n2 = o2 + l2;
-    double mag = hypot_pk(n1, n2);
-    if (mag > maxf)
-    {
-        n1 = n1 * (maxf / mag);
-        n2 = n2 * (maxf / mag);
-    }
-    t1.acc = n1;
-    t2.acc = n2;
-    double a1 = n1 - o1, a2 = n2 - o2;
-    if (!A.stat)
-    {
-        A.vel = A.vel + (t1.Jv * a1 + t2.Jv * a2) * A.im;
-        A.ang = A.ang + mul(A.Iwi, t1.Jwa * a1 + t2.Jwa * a2);
-    }
-    if (!B.stat)
-    {
-        B.vel = B.vel + ((-t1.Jv) * a1 - t2.Jv * a2) * B.im;
-        B.ang = B.ang + mul(B.Iwi, t1.Jwb * a1 + t2.Jwb * a2);
-    }
-}
-
-__device__ __forceinline__ void basis(v3 n, v3 &t1, v3 &t2) // :104-113
-{
-    double sign = copysign(1.0, n.z);
-    double a = -1.0 / (sign + n.z);
-    double b = n.x * n.y * a;
-    t1 = mk(1.0 + sign * n.x * n.x * a, sign * b, -sign * n.x);
-    t2 = mk(b, sign + n.y * n.y * a, -n.y);
-}
-
-__device__ __forceinline__ rowv make_row(const body_state &A, const body_state &B, v3 dir, v3 ra, v3 rb)
-{
-    rowv r;
-    r.Jv = dir;
-    r.Jwa = cross(ra, dir);
-    r.Jwb = -cross(rb, dir);
-    v3 ka = mul(A.Iwi, r.Jwa);
-    v3 kb = mul(B.Iwi, r.Jwb);
-    r.Meff = 1.0 / (((A.im + B.im) + dot(r.Jwa, ka)) + dot(r.Jwb, kb));
-    r.bias = 0.0;
-    r.acc = 0.0;
-    return r;
-}
 
 // Body velocities seen by a manifold solve: in device memory by body id (vel_global),
 // or in a workgroup's LDS table by slot for its dynamic bodies (vel_lds; static bodies,
@@ -169,18 +60,6 @@ struct vel_lds
     }
 };
 
-// inverse mass, inverse world inertia and the static flag (velocities come separately)
-__device__ __forceinline__ body_state ld_body(const bodies_dev &b, uint32_t i)
-{
-    body_state s;
-    s.vel = mk(0.0, 0.0, 0.0);
-    s.ang = mk(0.0, 0.0, 0.0);
-    s.im = b.inv_mass[i];
-    s.Iwi = ld9(b.Iw_inv, b.n, i);
-    s.stat = b.is_static[i] != 0;
-    return s;
-}
-
 // row field planes
 enum
 {
@@ -195,30 +74,11 @@ __device__ __forceinline__ double &rf(const rows_dev &r, int f, uint32_t slot)
 __device__ __forceinline__ v3 rf3(const rows_dev &r, int f, uint32_t slot)
 { return mk(rf(r, f, slot), rf(r, f + 1, slot), rf(r, f + 2, slot)); }
 
-// Contact c of manifold p: world normal n and lever arms as build_contact_jacobian
-// forms them (:883-890) and whether the contact makes rows (a penetration that is not
-// <= 0, so a NaN one does too, as in the reference's `if (penetration <= 0) continue`).
-__device__ __forceinline__ bool contact_frame(const manifolds_dev &m, uint32_t sl, int c, v3 pa, v3 pb, qt qa,
-                                              qt qb, v3 &n, v3 &ra, v3 &rb, double &pen)
-{
-    const double *d = m.data + static_cast<size_t>(c * kMF) * m.dcap + sl;
-    const size_t s = m.dcap;
-    const v3 nw = normalized(mk(d[0], d[s], d[2 * s]));
-    const v3 la = mk(d[3 * s], d[4 * s], d[5 * s]);
-    const v3 lb = mk(d[6 * s], d[7 * s], d[8 * s]);
-    const v3 lnb = rotate(conj(qb), nw);
-    ra = rotate(qa, la);
-    rb = rotate(qb, lb);
-    n = rotate(qb, lnb);
-    pen = dot((pb + rb) - (pa + ra), n);
-    return !(pen <= 0.0);
-}
-
 // which manifolds make solver rows: each is listed and its colour[p] set to kUncoloured
 // (no other pair's colour is read), and the row count; the rows themselves are written
 // by k_setup once the solve order is known
 __global__ void __launch_bounds__(kBlock)
-    k_row_flags(const uint64_t *keys, bodies_dev b, manifolds_dev m, uint32_t *colour, uint32_t *list,
+    k_row_flags(const uint64_t *keys, bodies_dev b, manifolds_dev m, uint32_t *colour, uint32_t *list, uint32_t *par,
                 unsigned long long *counters)
 {
     const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
@@ -238,7 +98,14 @@ __global__ void __launch_bounds__(kBlock)
             double pen;
             if (contact_frame(m, s, c, pa, pb, qa, qb, n, ra, rb, pen)) ++nrows;
         }
-        if (nrows) colour[p] = kUncoloured;
+        if (nrows)
+        {
+            colour[p] = kUncoloured;
+            // islands: the bodies of a row manifold belong together. A union that gave up
+            // (never seen; bounded so no thread can spin forever) makes the longest island
+            // all-ones, and the caller does without islands
+            if (par && !b.is_static[ia] && !b.is_static[ib] && !uf_union(par, ia, ib)) atomicMax(&counters[C_ISL_MAX], ~0ull);
+        }
     }
     block_add(&counters[C_ROWS], nrows);
     const unsigned long long at = block_append(&counters[C_NLIST], nrows > 0);
@@ -364,18 +231,6 @@ __global__ void __launch_bounds__(kBlock)
         }
     }
 }
-
-// Claim of a manifold in a colouring round: the round (from 1) above the complement of
-// mix32(p). mix32 is a bijection, so ordering by it equals ordering by the priority
-// (mix32(p) << 32) | p; an atomic max keeps this round's lowest priority at each body,
-// and claims left from earlier rounds lose to any claim of the current one, so the
-// claim array is cleared once per colouring, not every round.
-__device__ __forceinline__ uint64_t claim_of(uint32_t p, uint32_t round)
-{ return (static_cast<uint64_t>(round + 1u) << 32) | (0xFFFFFFFFu - mix32(p)); }
-
-__device__ __forceinline__ uint32_t local_index(uint32_t p, uint32_t ia, const uint32_t *world_of,
-                                                const uint32_t *pair_base)
-{ return pair_base ? p - pair_base[world_of[ia]] : p; }
 
 // first pair of each world in the sorted pair list (worlds without pairs are not written)
 __global__ void k_pair_base(const uint64_t *keys, uint32_t n_pairs, const uint32_t *world_of, uint32_t *pair_base)
@@ -543,17 +398,6 @@ __global__ void __launch_bounds__(kBlock)
 // Rows are computed in FP64 by k_setup<float> and stored once as FP32 in solve order;
 // the row arithmetic of the solve (J.v, lambda, clamping, the 2x2 friction block) runs
 // in FP32 and each body's velocity increment is added to its FP64 velocity.
-struct f3
-{
-    float x, y, z;
-};
-__device__ __forceinline__ f3 f3m(float x, float y, float z) { return {x, y, z}; }
-__device__ __forceinline__ f3 to_f3(v3 a) { return {static_cast<float>(a.x), static_cast<float>(a.y), static_cast<float>(a.z)}; }
-__device__ __forceinline__ float dotf(f3 a, f3 b) { return (a.x * b.x + a.y * b.y) + a.z * b.z; }
-__device__ __forceinline__ f3 scl(f3 a, float k) { return {a.x * k, a.y * k, a.z * k}; }
-__device__ __forceinline__ f3 addf(f3 a, f3 b) { return {a.x + b.x, a.y + b.y, a.z + b.z}; }
-__device__ __forceinline__ v3 widen(f3 a) { return mk(static_cast<double>(a.x), static_cast<double>(a.y), static_cast<double>(a.z)); }
-
 struct rows32_dev
 {
     uint32_t cap4;
@@ -581,8 +425,6 @@ struct body32
     float I[9];
     bool stat;
 };
-__device__ __forceinline__ f3 mulI(const float *I, f3 v)
-{ return f3m((I[0] * v.x + I[1] * v.y) + I[2] * v.z, (I[3] * v.x + I[4] * v.y) + I[5] * v.z, (I[6] * v.x + I[7] * v.y) + I[8] * v.z); }
 __device__ __forceinline__ body32 ld_body32(const bodies_dev &b, uint32_t i)
 {
     body32 s;
@@ -708,128 +550,29 @@ __global__ void k_writeback(const uint32_t *order, uint32_t n_act, manifolds_dev
     }
 }
 
-// ---- contact islands: connected components of the row manifolds over dynamic bodies ----
-// Union-find with hooking of the larger root under the smaller: every component's root
-// is its smallest body id, whatever order the unions run in.
-__device__ __forceinline__ uint32_t par_ld(uint32_t *par, uint32_t x)
-{ return __hip_atomic_load(&par[x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
-
-__device__ uint32_t uf_find(uint32_t *par, uint32_t x)
-{
-    uint32_t p = par_ld(par, x);
-    while (p != x)
-    {
-        uint32_t gp = par_ld(par, p);
-        if (gp != p) __hip_atomic_store(&par[x], gp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); // path halving
-        x = p;
-        p = gp;
-    }
-    return x;
-}
-
-__global__ void k_uf_init(uint32_t *par, uint32_t n)
-{
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) par[i] = i;
-}
-
-// the row manifolds are list[0..nl)
-__global__ void k_uf_union(const uint64_t *keys, const uint32_t *list, uint32_t nl, bodies_dev b, uint32_t *par)
-{
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nl) return;
-    const uint32_t p = list[i];
-    uint64_t key = keys[p];
-    uint32_t a = static_cast<uint32_t>(key >> 32), c = static_cast<uint32_t>(key & 0xFFFFFFFFu);
-    if (b.is_static[a] || b.is_static[c]) return;
-    for (uint32_t guard = 0; guard < 4096u; ++guard)
-    {
-        uint32_t ra = uf_find(par, a), rc = uf_find(par, c);
-        if (ra == rc) return;
-        uint32_t hi = ra > rc ? ra : rc, lo = ra > rc ? rc : ra;
-        uint32_t expect = hi;
-        if (__hip_atomic_compare_exchange_strong(&par[hi], &expect, lo, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
-                                                 __HIP_MEMORY_SCOPE_AGENT))
-            return;
-    }
-}
-
-__global__ void k_uf_flatten(uint32_t *par, uint32_t n)
-{
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) par[i] = uf_find(par, i);
-}
-
-// a union that gave up (never seen; bounded so no thread can spin forever) leaves two
-// bodies of one manifold in different islands: flagged, and the caller falls back
-__global__ void k_uf_verify(const uint64_t *keys, const uint32_t *list, uint32_t nl, bodies_dev b, const uint32_t *par,
-                            unsigned long long *fail)
-{
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nl) return;
-    const uint32_t p = list[i];
-    uint64_t key = keys[p];
-    uint32_t a = static_cast<uint32_t>(key >> 32), c = static_cast<uint32_t>(key & 0xFFFFFFFFu);
-    if (!b.is_static[a] && !b.is_static[c] && par[a] != par[c]) atomicMax(fail, ~0ull);
-}
-
+// ---- long contact islands ----
 // sort key of row manifold list[i]: (island root << cbits) | colour
-__global__ void k_island_keys(const uint64_t *keys, const uint32_t *colour, const uint32_t *list, uint32_t nl,
-                              bodies_dev b, const uint32_t *par, int cbits, uint64_t *out, uint32_t *vals)
+__global__ void k_island_keys(const uint32_t *colour, const uint32_t *list, uint32_t nl, const uint32_t *root_of,
+                              int cbits, uint64_t *out, uint32_t *vals)
 {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= nl) return;
     const uint32_t p = list[i];
-    const uint64_t key = keys[p];
-    uint32_t a = static_cast<uint32_t>(key >> 32);
-    if (b.is_static[a]) a = static_cast<uint32_t>(key & 0xFFFFFFFFu);
-    out[i] = (static_cast<uint64_t>(par[a]) << cbits) | colour[p];
+    out[i] = (static_cast<uint64_t>(root_of[i]) << cbits) | colour[p];
     vals[i] = p;
 }
 
-__global__ void k_island_flags(const uint64_t *sk, uint32_t n, uint64_t last, int cbits, uint32_t *flags)
+__global__ void k_island_flags(const uint64_t *sk, uint32_t n, int cbits, uint32_t *flags)
 {
     uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= n) return;
-    flags[t] = (sk[t] != last && (t == 0 || (sk[t] >> cbits) != (sk[t - 1] >> cbits))) ? 1u : 0u;
+    flags[t] = (t == 0 || (sk[t] >> cbits) != (sk[t - 1] >> cbits)) ? 1u : 0u;
 }
 
 __global__ void k_island_starts(const uint32_t *flags, const uint32_t *pos, uint32_t n, uint32_t *starts)
 {
     uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t < n && flags[t]) starts[pos[t]] = t;
-}
-
-// totals = (island count, row manifold count), read on the device; the grid covers an
-// upper bound of the island count
-__global__ void k_island_maxlen(const uint32_t *starts, const uint32_t *totals, unsigned long long *mx)
-{
-    const uint32_t n_isl = totals[0], n_act = totals[1];
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    uint32_t len = 0;
-    if (i < n_isl) len = (i + 1 < n_isl ? starts[i + 1] : n_act) - starts[i];
-    for (int off = 32; off > 0; off >>= 1)
-    {
-        uint32_t o = __shfl_xor(len, off);
-        len = o > len ? o : len;
-    }
-    if (__lane_id() == 0 && len) atomicMax(mx, static_cast<unsigned long long>(len));
-}
-
-// number of row manifolds: position of the first `last` key
-__global__ void k_count_below(const uint64_t *sk, uint32_t n, uint64_t last, uint32_t *out)
-{
-    if (blockIdx.x || threadIdx.x) return;
-    uint32_t lo = 0, hi = n;
-    while (lo < hi)
-    {
-        uint32_t mid = lo + ((hi - lo) >> 1);
-        if (sk[mid] < last)
-            lo = mid + 1;
-        else
-            hi = mid;
-    }
-    *out = lo;
 }
 
 // One workgroup per chunk of whole islands: chunk k holds the islands whose first
@@ -951,15 +694,6 @@ __device__ __forceinline__ void ctc_solve(ctc_t<double> &k, bool warm, body_stat
     k.a2 = t2.acc;
 }
 // FP32: solve_one32's arithmetic with the Jacobians rebuilt in FP32
-__device__ __forceinline__ f3 fcr(f3 a, f3 b) { return f3m(a.y * b.z - a.z * b.y, a.z * b.x - a.x * b.z, a.x * b.y - a.y * b.x); }
-__device__ __forceinline__ void fbasis(f3 n, f3 &t1, f3 &t2)
-{
-    const float sign = copysignf(1.0f, n.z);
-    const float a = -1.0f / (sign + n.z);
-    const float b = n.x * n.y * a;
-    t1 = f3m(1.0f + sign * n.x * n.x * a, sign * b, -sign * n.x);
-    t2 = f3m(b, sign + n.y * n.y * a, -n.y);
-}
 __device__ __forceinline__ void ctc_solve(ctc_t<float> &k, bool warm, body32 &A, body32 &B)
 {
     const f3 n = f3m(k.n[0], k.n[1], k.n[2]), ra = f3m(k.ra[0], k.ra[1], k.ra[2]), rb = f3m(k.rb[0], k.rb[1], k.rb[2]);
@@ -1081,8 +815,9 @@ __device__ __forceinline__ void solve_chunk_reg(const uint64_t *keys, const uint
 // sized to match) halves the LDS, and its FP32 form is held to two waves per SIMD, so
 // two workgroups share a CU; CAP 512 keeps every register for its long islands.
 constexpr int kIslandThreads = 256;
-template <bool F32, int CAP>
-__global__ void __launch_bounds__(kIslandThreads, (F32 && CAP == 256) ? 2 : 1)
+constexpr int CAP = 2 * kIslandThreads;
+template <bool F32>
+__global__ void __launch_bounds__(kIslandThreads)
     k_solve_islands(const uint64_t *keys, const uint32_t *order, const uint64_t *sk, const uint32_t *starts,
                     uint32_t n_isl, uint32_t n_act, uint32_t n_colours, int cbits, bodies_dev b, rows_dev r,
                     uint32_t cap, uint32_t iters, uint32_t window)
@@ -1201,10 +936,10 @@ __global__ void __launch_bounds__(kIslandThreads, (F32 && CAP == 256) ? 2 : 1)
 } // namespace
 
 void launch_row_flags(const uint64_t *keys, uint32_t n_pairs, const bodies_dev &b, manifolds_dev m, uint32_t *colour,
-                      uint32_t *list, unsigned long long *counters, hipStream_t st)
+                      uint32_t *list, uint32_t *par, unsigned long long *counters, hipStream_t st)
 {
     if (!n_pairs) return;
-    if (m.dcap) k_row_flags<<<grid(m.dcap), kBlock, 0, st>>>(keys, b, m, colour, list, counters);
+    if (m.dcap) k_row_flags<<<grid(m.dcap), kBlock, 0, st>>>(keys, b, m, colour, list, par, counters);
 }
 void launch_contact_setup(const uint64_t *keys, uint32_t n, const uint32_t *ord, uint32_t cap, const bodies_dev &b,
                           manifolds_dev m, rows_dev r, double dt, double threshold, bool f32, hipStream_t st)
@@ -1267,24 +1002,17 @@ void launch_impulse_writeback(const uint32_t *order, uint32_t n_act, manifolds_d
 }
 
 island_sort launch_island_sort(const uint64_t *keys, const uint32_t *colour, const uint32_t *list, uint32_t nl,
-                               uint32_t n_colours, const bodies_dev &b, uint32_t *par, uint64_t *ik, uint32_t *iv,
-                               uint64_t *ik_alt, uint32_t *iv_alt, unsigned long long *fail, sort_scratch &sc,
-                               hipStream_t st)
+                               uint32_t n_colours, uint32_t n_bodies, const uint32_t *root_of, uint64_t *ik, uint32_t *iv,
+                               uint64_t *ik_alt, uint32_t *iv_alt, sort_scratch &sc, hipStream_t st)
 {
     island_sort is{};
-    const uint32_t n = b.n;
-    k_uf_init<<<grid(n), kBlock, 0, st>>>(par, n);
-    if (nl) k_uf_union<<<grid(nl), kBlock, 0, st>>>(keys, list, nl, b, par);
-    k_uf_flatten<<<grid(n), kBlock, 0, st>>>(par, n);
-    if (nl) k_uf_verify<<<grid(nl), kBlock, 0, st>>>(keys, list, nl, b, par, fail);
     int cbits = 1;
     while (cbits < 31 && (1u << cbits) <= n_colours) ++cbits;
     int ibits = 1;
-    while (ibits < 32 && (1ull << ibits) < n) ++ibits;
+    while (ibits < 32 && (1ull << ibits) < n_bodies) ++ibits;
     const int bits = cbits + ibits;
     is.cbits = cbits;
-    is.last = (1ull << bits) - 1;
-    if (nl) k_island_keys<<<grid(nl), kBlock, 0, st>>>(keys, colour, list, nl, b, par, cbits, ik, iv);
+    if (nl) k_island_keys<<<grid(nl), kBlock, 0, st>>>(colour, list, nl, root_of, cbits, ik, iv);
     int shifts[8];
     int ns = 0;
     for (int sft = 0; sft < bits; sft += 8) shifts[ns++] = sft;
@@ -1293,41 +1021,26 @@ island_sort launch_island_sort(const uint64_t *keys, const uint32_t *colour, con
     is.ord = alt ? iv_alt : iv;
     return is;
 }
-void launch_island_segments(const island_sort &is, uint32_t n_pairs, uint32_t *flags, uint32_t *pos, uint32_t *bsums,
-                            uint32_t *total, uint32_t *starts, uint32_t *n_act, hipStream_t st)
+void launch_island_segments(const island_sort &is, uint32_t nl, uint32_t *flags, uint32_t *pos, uint32_t *bsums,
+                            uint32_t *total, uint32_t *starts, hipStream_t st)
 {
-    k_count_below<<<1, 64, 0, st>>>(is.sk, n_pairs, is.last, n_act);
-    k_island_flags<<<grid(n_pairs), kBlock, 0, st>>>(is.sk, n_pairs, is.last, is.cbits, flags);
-    exclusive_scan_u32(flags, pos, n_pairs, bsums, total, st);
-    k_island_starts<<<grid(n_pairs), kBlock, 0, st>>>(flags, pos, n_pairs, starts);
-}
-void launch_island_maxlen(const uint32_t *starts, const uint32_t *totals, uint32_t max_islands,
-                          unsigned long long *mx, hipStream_t st)
-{
-    if (max_islands) k_island_maxlen<<<grid(max_islands), kBlock, 0, st>>>(starts, totals, mx);
+    k_island_flags<<<grid(nl), kBlock, 0, st>>>(is.sk, nl, is.cbits, flags);
+    exclusive_scan_u32(flags, pos, nl, bsums, total, st);
+    k_island_starts<<<grid(nl), kBlock, 0, st>>>(flags, pos, nl, starts);
 }
 void launch_solve_islands(const uint64_t *keys, const island_sort &is, const uint32_t *starts, uint32_t n_isl,
                           uint32_t n_act, uint32_t n_colours, const bodies_dev &b, const rows_dev &r, uint32_t cap,
-                          uint32_t iters, uint32_t longest, bool f32, hipStream_t st)
+                          uint32_t iters, bool f32, hipStream_t st)
 {
     if (!n_isl) return;
-    // the smaller workgroup (and LDS) when every island fits it, so more chunks are
-    // resident at once; windows shrink with the longest island so every chunk fits
-    auto go = [&](auto capacity, uint32_t window)
-    {
-        constexpr int CAP = decltype(capacity)::value;
-        const unsigned nb = static_cast<unsigned>((n_act + window - 1) / window);
-        if (f32)
-            k_solve_islands<true, CAP><<<nb, kIslandThreads, 0, st>>>(keys, is.ord, is.sk, starts, n_isl, n_act,
-                                                                       n_colours, is.cbits, b, r, cap, iters, window);
-        else
-            k_solve_islands<false, CAP><<<nb, kIslandThreads, 0, st>>>(keys, is.ord, is.sk, starts, n_isl, n_act,
-                                                                        n_colours, is.cbits, b, r, cap, iters, window);
-    };
-    if (longest <= static_cast<uint32_t>(kIslandThreads))
-        go(std::integral_constant<int, kIslandThreads>{}, kIslandThreads + 1 - std::max<uint32_t>(longest, 1));
+    constexpr uint32_t window = kIslandThreads;
+    const unsigned nb = static_cast<unsigned>((n_act + window - 1) / window);
+    if (f32)
+        k_solve_islands<true><<<nb, kIslandThreads, 0, st>>>(keys, is.ord, is.sk, starts, n_isl, n_act, n_colours, is.cbits,
+                                                             b, r, cap, iters, window);
     else
-        go(std::integral_constant<int, 2 * kIslandThreads>{}, kIslandThreads);
+        k_solve_islands<false><<<nb, kIslandThreads, 0, st>>>(keys, is.ord, is.sk, starts, n_isl, n_act, n_colours, is.cbits,
+                                                              b, r, cap, iters, window);
 }
 void launch_solve_colour32(const uint64_t *keys, const uint32_t *order, uint32_t begin, uint32_t end,
                            const bodies_dev &b, rows_dev r32, uint32_t cap, bool warm, hipStream_t st)

@@ -78,7 +78,7 @@ enum counter_slot
 {
     C_MOVED = 0,
     C_CAND = 1,
-    // 2: unused
+    C_ISL_CUR = 2, // positions given to contact islands
     C_PAIRS = 3,
     C_HITS = 4,
     C_CONTACTS = 5,
@@ -370,12 +370,13 @@ struct rows_dev
 constexpr int kRowF = 44; // 38 row words + the contact's lever arms (6)
 constexpr uint32_t kUncoloured = 0xFFFFFFFEu; // colour of an item still to be coloured
 // colour[p] = kUncoloured for manifolds that make solver rows (else kNone), their row
-// count at counters[C_ROWS], and those manifolds listed in list (count in C_NLIST).
+// count at counters[C_ROWS], and those manifolds listed in list (count in C_NLIST); with
+// par, their bodies united into islands (k_island.hip).
 // Only pairs holding contacts can make rows: the pass runs over the data slots the
 // manifold update filled (counters[C_MSLOTS] of at most m.dcap) after every colour has
 // been set to kNone.
 void launch_row_flags(const uint64_t *keys, uint32_t n_pairs, const bodies_dev &b, manifolds_dev m, uint32_t *colour,
-                      uint32_t *list, unsigned long long *counters, hipStream_t st);
+                      uint32_t *list, uint32_t *par, unsigned long long *counters, hipStream_t st);
 // rows of manifold ord[k], k < n, at slots c * cap + k of r (solve order); with ord
 // null, of manifold k at slots 4k + c (pair order). f32: r.d holds FP32 planes (the
 // rows computed in FP64 and rounded once)
@@ -409,34 +410,51 @@ void launch_solve_colour(const uint64_t *keys, const uint32_t *order, uint32_t b
                          const bodies_dev &b, rows_dev r, uint32_t cap, bool warm, hipStream_t st);
 void launch_impulse_writeback(const uint32_t *order, uint32_t n_act, manifolds_dev m, rows_dev r, uint32_t cap,
                               hipStream_t st);
-// Contact islands (connected components of the row manifolds over dynamic bodies,
-// each rooted at its smallest body id), manifolds sorted by (island, colour): a
+// ---------------- k_island.hip ----------------
+// Contact islands: connected components of the row manifolds over dynamic bodies, each
+// rooted at its smallest body id. launch_island_init before launch_row_flags (which unites
+// the bodies of each row manifold), then the roots: manifolds per root in cnt, each listed
+// manifold's root and rank, the longest island in counters[C_ISL_MAX] (all-ones if a union
+// gave up).
+void launch_island_init(uint32_t *par, uint32_t *cnt, uint32_t n, hipStream_t st);
+void launch_island_roots(const uint64_t *keys, const uint32_t *list, uint32_t n_bound, const bodies_dev &b, uint32_t *par,
+                         uint32_t *cnt, uint32_t *root_of, uint32_t *rank_of, unsigned long long *counters, hipStream_t st);
+// the listed manifolds with every island's together (ord), and each position's root (isl);
+// base: n_bodies entries of scratch
+void launch_island_group(const uint32_t *list, uint32_t nl, const uint32_t *cnt, uint32_t n_bodies, const uint32_t *root_of,
+                         const uint32_t *rank_of, uint32_t *base, uint32_t *ord, uint32_t *isl,
+                         unsigned long long *counters, hipStream_t st);
+// The whole contact solve of islands of at most kChunkMax manifolds (kChunkMax32 for the FP32
+// solve, whose longer islands keep the row arithmetic of launch_solve_islands). isl null: the
+// list (at most kChunkTwoLanes) is one chunk. Two lanes per manifold up to 256 manifolds: 512
+// threads, the most whose FP64 rows of four contacts fit the 256 registers a thread then has;
+// one lane, with its lever arms in LDS, up to 512.
+constexpr int kChunkTwoLanes = 256, kChunkMax = 512, kChunkMax32 = 256;
+constexpr uint32_t kChunkFill = 32; // manifolds a chunk takes before another workgroup is opened
+void launch_solve_chunks(const uint64_t *keys, const uint32_t *ord, const uint32_t *isl, uint32_t nl, uint32_t longest,
+                         const bodies_dev &b, const manifolds_dev &m, uint32_t *colour, const uint32_t *world_of,
+                         const uint32_t *pair_base, uint32_t iters, double dt, double thr, bool f32,
+                         unsigned long long *counters, hipStream_t st);
+// Longer islands (up to kIslandMaxManifolds), manifolds sorted by (island, colour): a
 // workgroup solves a chunk of whole islands, every colour and pass, in one launch.
 struct island_sort
 {
-    const uint64_t *sk;  // sorted keys (island << cbits | colour; `last` for no rows)
+    const uint64_t *sk;  // sorted keys (island << cbits | colour)
     const uint32_t *ord; // manifold index at each sorted position
     int cbits;
-    uint64_t last;
 };
 constexpr uint32_t kIslandMaxManifolds = 4096; // larger islands use the per-colour launches
 constexpr uint32_t kIslandMaxColours = 64;  // above: the per-colour launches
-// `fail` becomes all-ones if the islands could not be built (the caller then falls back)
-// over the nl row manifolds list[0..nl) (the colouring's list); positions of the sorted
-// order index that list's manifolds, so n_pairs below is nl
+// over the nl row manifolds list[0..nl), whose roots are root_of
 island_sort launch_island_sort(const uint64_t *keys, const uint32_t *colour, const uint32_t *list, uint32_t nl,
-                               uint32_t n_colours, const bodies_dev &b, uint32_t *par, uint64_t *ik, uint32_t *iv,
-                               uint64_t *ik_alt, uint32_t *iv_alt, unsigned long long *fail, sort_scratch &sc,
-                               hipStream_t st);
-// island starts (positions where the island changes) and the row-manifold count
-void launch_island_segments(const island_sort &is, uint32_t n_pairs, uint32_t *flags, uint32_t *pos, uint32_t *bsums,
-                            uint32_t *total, uint32_t *starts, uint32_t *n_act, hipStream_t st);
-void launch_island_maxlen(const uint32_t *starts, const uint32_t *totals, uint32_t max_islands,
-                          unsigned long long *mx, hipStream_t st);
-// longest: manifolds of the longest island (chunks are sized so each fits one workgroup)
+                               uint32_t n_colours, uint32_t n_bodies, const uint32_t *root_of, uint64_t *ik, uint32_t *iv,
+                               uint64_t *ik_alt, uint32_t *iv_alt, sort_scratch &sc, hipStream_t st);
+// island starts (positions where the island changes) and their number
+void launch_island_segments(const island_sort &is, uint32_t nl, uint32_t *flags, uint32_t *pos, uint32_t *bsums,
+                            uint32_t *total, uint32_t *starts, hipStream_t st);
 void launch_solve_islands(const uint64_t *keys, const island_sort &is, const uint32_t *starts, uint32_t n_isl,
                           uint32_t n_act, uint32_t n_colours, const bodies_dev &b, const rows_dev &r, uint32_t cap,
-                          uint32_t iters, uint32_t longest, bool f32, hipStream_t st);
+                          uint32_t iters, bool f32, hipStream_t st);
 // FP32 solve (rows_dev whose d holds FP32 planes, written by launch_contact_setup with
 // f32; body velocities accumulate in FP64)
 void launch_solve_colour32(const uint64_t *keys, const uint32_t *order, uint32_t begin, uint32_t end,
