@@ -17,6 +17,8 @@
 #include <mutex>
 #include <stdexcept>
 #include <string>
+#include <system_error>
+#include <thread>
 #include <vector>
 
 namespace
@@ -100,6 +102,66 @@ __global__ void k_set_state(bodies_dev b, uint32_t count, const uint32_t *ids, c
     }
 }
 
+// Bodies [first, first + count) as the caller's arrays hold them (one record per body), each
+// array's part at its pointer: a thread per 8-byte word, so stores are contiguous
+struct export_to
+{
+    double *pos, *vel, *ang, *quat, *fat;
+    uint8_t *moved;
+};
+__global__ void k_export(bodies_dev b, uint32_t first, uint32_t count, export_to o)
+{
+    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+    auto records = [&](double *dst, const double *planes, uint32_t k)
+    {
+        if (dst && t < k * count) dst[t] = planes[static_cast<size_t>(t % k) * b.n + first + t / k];
+    };
+    records(o.pos, b.pos, 3);
+    records(o.vel, b.vel, 3);
+    records(o.ang, b.ang, 3);
+    records(o.quat, b.quat, 4);
+    if (o.fat && t < 6 * count) o.fat[t] = b.fat[6 * static_cast<size_t>(first) + t];
+    if (o.moved && t < count) o.moved[t] = b.moved[first + t];
+}
+
+// host memory parts copied together, split over a few threads when large (a fresh array's
+// pages are faulted in by whoever writes them first)
+struct host_part
+{
+    char *dst;
+    const char *src;
+    size_t bytes;
+};
+void copy_parts(const std::vector<host_part> &parts)
+{
+    size_t total = 0;
+    for (const host_part &p : parts) total += p.bytes;
+    auto range = [&](size_t lo, size_t hi)
+    {
+        size_t at = 0;
+        for (const host_part &p : parts)
+        {
+            const size_t a = std::max(lo, at), e = std::min(hi, at + p.bytes);
+            if (a < e) std::memcpy(p.dst + (a - at), p.src + (a - at), e - a);
+            at += p.bytes;
+        }
+    };
+    const size_t n = std::min<size_t>(std::min<size_t>(8, std::thread::hardware_concurrency()), total >> 20);
+    if (n < 2) return range(0, total);
+    std::vector<std::thread> team;
+    team.reserve(n - 1);
+    size_t done = 0; // the parts given to threads; the rest, also after a thread could not start, is copied here
+    try
+    {
+        for (; done + 1 < n; ++done) team.emplace_back(range, total / n * done, total / n * (done + 1));
+    }
+    catch (const std::system_error &)
+    {
+    }
+    range(total / n * done, total);
+    for (std::thread &t : team) t.join();
+}
+
 int id_bits(uint32_t n)
 {
     int b = 0;
@@ -122,11 +184,6 @@ std::vector<double> planar(const double *a, uint32_t n, int k)
     for (uint32_t i = 0; i < n; ++i)
         for (int c = 0; c < k; ++c) o[static_cast<size_t>(c) * n + i] = a[static_cast<size_t>(i) * k + c];
     return o;
-}
-void aos(const std::vector<double> &p, uint32_t n, int k, double *out)
-{
-    for (uint32_t i = 0; i < n; ++i)
-        for (int c = 0; c < k; ++c) out[static_cast<size_t>(i) * k + c] = p[static_cast<size_t>(c) * n + i];
 }
 template <class T> std::vector<T> download(const dbuf<T> &d, size_t count, hipStream_t st)
 {
@@ -284,6 +341,14 @@ struct pkg_ctx
     dbuf<uint32_t> q_out_id, q_world;
     hipEvent_t q_ev[2] = {nullptr, nullptr}; // query kernel timing
 
+    // body state on its way between the caller's arrays and the device: two halves of pinned
+    // memory and of device memory, grown on use up to kXferHalf each, kept until the ctx ends
+    char *xfer_pin = nullptr;
+    size_t xfer_half = 0;
+    dbuf<char> xfer_dev;
+    hipEvent_t xfer_ev[2] = {nullptr, nullptr};
+    void xfer_reserve(size_t bytes);
+
     pkg_counters last{};
     bool have_bodies = false;
     // a step failed part-way: body state holds part of that step, so stepping is refused
@@ -432,6 +497,26 @@ void record(hipEvent_t *ev, int k, hipStream_t st)
     if (ev) hip_check(hipEventRecord(ev[k], st), "event record");
 }
 } // namespace
+
+// Up to this many bytes of body state the kernels read and write the pinned memory
+// themselves (one launch and one wait: 64 bodies downloaded in 0.03 ms); more goes through
+// device memory and the copy engine in halves, the host's copy of one half overlapping the
+// transfer of the other.
+constexpr size_t kXferDirect = 256 << 10, kXferHalf = 16 << 20;
+void pkg_ctx::xfer_reserve(size_t bytes)
+{
+    for (auto &e : xfer_ev)
+        if (!e) hip_check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "event create");
+    if (bytes > kXferDirect) xfer_dev.reserve(2 * kXferHalf);
+    size_t half = kXferDirect;
+    if (bytes > half) half = kXferHalf;
+    if (half <= xfer_half) return;
+    if (xfer_pin) (void)hipHostFree(xfer_pin);
+    xfer_pin = nullptr;
+    xfer_half = 0;
+    hip_check(hipHostMalloc(reinterpret_cast<void **>(&xfer_pin), 2 * half), "pinned alloc");
+    xfer_half = half;
+}
 
 lbvh_dev pkg_ctx::tree()
 {
@@ -1234,6 +1319,9 @@ pkg_status pkg_destroy(pkg_ctx *ctx)
     if (ctx->sc.hist) (void)hipFree(ctx->sc.hist);
     for (hipEvent_t e : ctx->q_ev)
         if (e) (void)hipEventDestroy(e);
+    for (hipEvent_t e : ctx->xfer_ev)
+        if (e) (void)hipEventDestroy(e);
+    if (ctx->xfer_pin) (void)hipHostFree(ctx->xfer_pin);
     if (ctx->h_counters) (void)hipHostFree(ctx->h_counters);
     if (ctx->st) (void)hipStreamDestroy(ctx->st);
     delete ctx;
@@ -1745,23 +1833,45 @@ pkg_status pkg_set_body_state(pkg_ctx *ctx, uint32_t count, const uint32_t *ids,
     PKG_GUARD(ctx, {
         if (!count) return PKG_OK;
         hipStream_t st = ctx->st;
-        dbuf<uint32_t> di;
-        dbuf<double> dp, dv, da, dq;
-        upload(di, ids, count, st);
-        if (pos) upload(dp, pos, 3 * static_cast<size_t>(count), st);
-        if (vel) upload(dv, vel, 3 * static_cast<size_t>(count), st);
-        if (angvel) upload(da, angvel, 3 * static_cast<size_t>(count), st);
-        if (quat) upload(dq, quat, 4 * static_cast<size_t>(count), st);
-        k_set_state<<<(count + 255) / 256, 256, 0, st>>>(ctx->B(), count, di.p, pos ? dp.p : nullptr,
-                                                         vel ? dv.p : nullptr, angvel ? da.p : nullptr,
-                                                         quat ? dq.p : nullptr);
-        hip_check(hipGetLastError(), "set state launch");
+        const double *src[4] = {pos, vel, angvel, quat};
+        const size_t width[4] = {24, 24, 24, 32}; // bytes per body
+        size_t rec = 4;
+        for (int a = 0; a < 4; ++a)
+            if (src[a]) rec += width[a];
+        ctx->xfer_reserve(rec * count);
+        const bool direct = rec * count <= kXferDirect;
+        // records per half, a multiple of 64 so every array of a half starts aligned
+        const uint32_t per = direct ? count : static_cast<uint32_t>(std::min<size_t>(kXferHalf / rec / 64 * 64, count));
+        for (uint32_t first = 0, round = 0; first < count; first += per, ++round)
+        {
+            const uint32_t n = std::min(per, count - first), h = round & 1;
+            // the half's last transfer has left the pinned memory
+            if (round > 1) hip_check(hipEventSynchronize(ctx->xfer_ev[h]), "event sync");
+            char *pin = ctx->xfer_pin + h * ctx->xfer_half;
+            char *dev = direct ? pin : ctx->xfer_dev.p + h * kXferHalf;
+            std::vector<host_part> parts;
+            const double *d[4] = {};
+            size_t at = 0;
+            for (int a = 0; a < 4; ++a)
+                if (src[a])
+                {
+                    parts.push_back({pin + at, reinterpret_cast<const char *>(src[a]) + width[a] * first, width[a] * n});
+                    d[a] = reinterpret_cast<const double *>(dev + at);
+                    at += width[a] * n;
+                }
+            const uint32_t *di = reinterpret_cast<const uint32_t *>(dev + at);
+            parts.push_back({pin + at, reinterpret_cast<const char *>(ids + first), 4 * static_cast<size_t>(n)});
+            at += 4 * static_cast<size_t>(n);
+            copy_parts(parts);
+            if (!direct)
+            {
+                hip_check(hipMemcpyAsync(dev, pin, at, hipMemcpyHostToDevice, st), "state copy");
+                hip_check(hipEventRecord(ctx->xfer_ev[h], st), "event record");
+            }
+            k_set_state<<<(n + 255) / 256, 256, 0, st>>>(ctx->B(), n, di, d[0], d[1], d[2], d[3]);
+            hip_check(hipGetLastError(), "set state launch");
+        }
         hip_check(hipStreamSynchronize(st), "set state");
-        di.release();
-        dp.release();
-        dv.release();
-        da.release();
-        dq.release();
     })
 }
 
@@ -1933,27 +2043,54 @@ pkg_status pkg_download_bodies(pkg_ctx *ctx, const pkg_body_state *out)
 {
     if (!ctx || !out) return PKG_INVALID_ARG;
     PKG_GUARD(ctx, {
-        uint32_t n = ctx->n;
+        const uint32_t n = ctx->n;
         hipStream_t st = ctx->st;
-        auto get = [&](dbuf<double> &b, int k, double *dst)
+        void *dst[6] = {out->pos, out->vel, out->angvel, out->quat, out->fat, out->moved};
+        const size_t width[6] = {24, 24, 24, 32, 48, 1}; // bytes per body
+        size_t rec = 0;
+        for (int a = 0; a < 6; ++a)
+            if (dst[a]) rec += width[a];
+        if (!n || !rec) return PKG_OK;
+        ctx->xfer_reserve(rec * n);
+        const bool direct = rec * n <= kXferDirect;
+        const uint32_t per = direct ? n : static_cast<uint32_t>(std::min<size_t>(kXferHalf / rec / 64 * 64, n));
+        std::vector<host_part> parts[2];
+        const uint32_t rounds = (n + per - 1) / per;
+        for (uint32_t round = 0; round <= rounds; ++round)
         {
-            if (!dst) return;
-            std::vector<double> h = download(b, static_cast<size_t>(n) * k, st);
-            aos(h, n, k, dst);
-        };
-        get(ctx->pos, 3, out->pos);
-        get(ctx->vel, 3, out->vel);
-        get(ctx->ang, 3, out->angvel);
-        get(ctx->quat, 4, out->quat);
-        if (out->fat) // already one record per body
-        {
-            std::vector<double> h = download(ctx->fat, static_cast<size_t>(n) * 6, st);
-            std::memcpy(out->fat, h.data(), h.size() * sizeof(double));
-        }
-        if (out->moved)
-        {
-            std::vector<uint8_t> m = download(ctx->moved, n, st);
-            std::memcpy(out->moved, m.data(), n);
+            if (round < rounds)
+            {
+                const uint32_t first = round * per, count = std::min(per, n - first), h = round & 1;
+                char *pin = ctx->xfer_pin + h * ctx->xfer_half;
+                char *dev = direct ? pin : ctx->xfer_dev.p + h * kXferHalf;
+                char *to[6] = {};
+                size_t at = 0;
+                parts[h].clear();
+                for (int a = 0; a < 6; ++a)
+                    if (dst[a])
+                    {
+                        to[a] = dev + at;
+                        parts[h].push_back({static_cast<char *>(dst[a]) + width[a] * first, pin + at, width[a] * count});
+                        at += width[a] * count;
+                    }
+                export_to o;
+                o.pos = reinterpret_cast<double *>(to[0]);
+                o.vel = reinterpret_cast<double *>(to[1]);
+                o.ang = reinterpret_cast<double *>(to[2]);
+                o.quat = reinterpret_cast<double *>(to[3]);
+                o.fat = reinterpret_cast<double *>(to[4]);
+                o.moved = reinterpret_cast<uint8_t *>(to[5]);
+                k_export<<<(6 * count + 255) / 256, 256, 0, st>>>(ctx->B(), first, count, o);
+                hip_check(hipGetLastError(), "export launch");
+                if (!direct) hip_check(hipMemcpyAsync(pin, dev, at, hipMemcpyDeviceToHost, st), "state copy");
+                hip_check(hipEventRecord(ctx->xfer_ev[h], st), "event record");
+            }
+            if (round > 0) // the half before, while this one is on its way
+            {
+                const uint32_t h = (round - 1) & 1;
+                hip_check(hipEventSynchronize(ctx->xfer_ev[h]), "event sync");
+                copy_parts(parts[h]);
+            }
         }
     })
 }
