@@ -607,6 +607,12 @@ __global__ void __launch_bounds__(kBlock) k_span(lbvh_dev t)
 // large scenes workgroups write to several regions with a cursor each and reserve per
 // wavefront, so no wavefront waits for its workgroup's longest walk.
 constexpr int kEmitBuf = 32;
+// Up to this many leaves kSlices threads share a query; beyond it the chip is full without
+// and the extra walks' first steps only add work. Pair stage with 1, 8 and 16 slices: boxes
+// 16,385 leaves 0.54, 0.38 and 0.34 ms, batched worlds 10,000 0.235, 0.179 and 0.172, hulls
+// 16,384 0.272, 0.257 and 0.260, 32,768 0.297, 0.302 and 0.308, 131,072 0.40, 0.57 and 0.74.
+constexpr uint32_t kSliceLeaves = 24576;
+constexpr uint32_t kSlices = 16;
 
 // The node whose leaf range is exactly [lo, hi]: a world's leaves share the world bits
 // at the top of their keys, so they form one subtree, whose root (a Karras node sits at
@@ -628,6 +634,12 @@ __device__ __forceinline__ void flush_own(uint64_t *buf, uint32_t cnt, uint64_t 
         if (base + k < cap) out_keys[base + k] = buf[k];
 }
 
+// A walk is a chain of dependent node loads (about 0.4 us each), so with few leaves the
+// longest walk bounds the kernel. SLICED: kSlices threads share a query, each walking the
+// subtrees of its slice of the world's leaves: from the slice's first leaf through the
+// escape links, a rejected node skipping past its last leaf, until the next leaf is the
+// next slice's. 1,024 boxes: pair stage 0.265 -> 0.161 ms.
+template <bool SLICED>
 __global__ void __launch_bounds__(kBlock)
     k_pair_query(lbvh_dev t, bodies_dev b, uint64_t *regions, uint32_t cap, uint32_t n_regions,
                  unsigned long long *counters)
@@ -640,7 +652,9 @@ __global__ void __launch_bounds__(kBlock)
     // thread k walks for the k-th moved leaf (sorted index i), list blocks in XCD order
     const uint32_t n = t.n;
     const uint32_t n_moved = static_cast<uint32_t>(counters[C_MLEAF]);
-    const uint32_t k = xcd_block(n_moved, blockDim.x) * blockDim.x + threadIdx.x;
+    const uint64_t items = SLICED ? static_cast<uint64_t>(n_moved) * kSlices : n_moved;
+    const uint32_t item = xcd_block(items, blockDim.x) * blockDim.x + threadIdx.x;
+    const uint32_t k = SLICED ? item / kSlices : item;
     const uint32_t i = k < n_moved ? t.moved_list[k] : n;
     bool active = false;
     uint32_t a = 0;
@@ -671,16 +685,27 @@ __global__ void __launch_bounds__(kBlock)
         uint32_t w = t.world_of[a];
         wlo = t.wstart[w];
         whi = t.wstart[w + 1] - 1;
-        const uint32_t root = range_root(t, wlo, whi);
-        if (root != kNone)
+        if (!SLICED)
         {
-            node = root;
-            stop = t.escape[root];
+            const uint32_t root = range_root(t, wlo, whi);
+            if (root != kNone)
+            {
+                node = root;
+                stop = t.escape[root];
+            }
+            else
+                ranged = true;
         }
-        else
-            ranged = true;
     }
-    for (uint32_t guard = 0; node != stop; ++guard)
+    uint32_t at = 0, end = 0; // SLICED: the first leaf below `node`, the slice's end
+    if (SLICED && active)
+    {
+        const uint32_t len = whi - wlo + 1, s = item % kSlices;
+        at = wlo + static_cast<uint32_t>(static_cast<uint64_t>(len) * s / kSlices);
+        end = wlo + static_cast<uint32_t>(static_cast<uint64_t>(len) * (s + 1) / kSlices);
+        node = at < end ? n - 1 + at : kNone;
+    }
+    for (uint32_t guard = 0; node != stop && (!SLICED || at < end); ++guard)
     {
         if (guard >= 2 * n)
         {
@@ -694,18 +719,22 @@ __global__ void __launch_bounds__(kBlock)
             bool ov = lo.x <= qhi[0] && hi.x >= qlo[0] && lo.y <= qhi[1] && hi.y >= qlo[1] && lo.z <= qhi[2] &&
                       hi.z >= qlo[2];
             next = __float_as_uint(hi.w);
-            if (ov && ranged) ov = t.first[node] <= whi && (t.lastf[node] & 0x7fffffffu) >= wlo;
-            if (ov)
+            if (!SLICED && ov && ranged) ov = t.first[node] <= whi && (t.lastf[node] & 0x7fffffffu) >= wlo;
+            if (SLICED || ov)
             {
                 uint32_t lf = t.lastf[node];
                 bool skip = (lf & 0x7fffffffu) <= i && (lf >> 31);
-                if (!skip) next = __float_as_uint(lo.w);
+                if (ov && !skip)
+                    next = __float_as_uint(lo.w);
+                else
+                    at = (lf & 0x7fffffffu) + 1;
             }
         }
         else
         {
             uint32_t j = node - (n - 1);
             next = t.escape[node];
+            at = j + 1;
             bool near = j != i && j >= wlo && j <= whi;
             bool sure = false;
             if (near && t.leaf_f32)
@@ -916,7 +945,11 @@ void launch_pair_query(const lbvh_dev &t, const bodies_dev &b, uint64_t *out_key
 {
     if (t.n < 2) return;
     // a multiple of 8 workgroups, so every XCD's eighth of the list has its workgroups
-    k_pair_query<<<(grid(t.n) + 7) / 8 * 8, kBlock, 0, st>>>(t, b, out_keys, cap, n_regions, counters);
+    auto wgs = [](size_t threads) { return (grid(threads) + 7) / 8 * 8; };
+    if (t.n <= kSliceLeaves)
+        k_pair_query<true><<<wgs(static_cast<size_t>(t.n) * kSlices), kBlock, 0, st>>>(t, b, out_keys, cap, n_regions, counters);
+    else
+        k_pair_query<false><<<wgs(t.n), kBlock, 0, st>>>(t, b, out_keys, cap, n_regions, counters);
 }
 
 void launch_pair_match(const uint64_t *cand, uint32_t m, const uint64_t *prev, uint32_t n_prev, uint32_t *src,
