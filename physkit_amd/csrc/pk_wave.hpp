@@ -11,7 +11,13 @@
 //   - the silhouette walk (a few scalar instructions per visible face), the heap's path
 //     and the lists' counts are uniform, in scalar registers;
 //   - the new faces of an expansion are built one per lane;
-//   - a heap push or pop compares its whole path at once (one LDS round trip).
+//   - the nearest face is a minimum over the registers. The heap that the one-thread solver
+//     keeps only decides between live faces at the same distance: the first time it has
+//     to, it is built by repeating its pushes and pops so far, and kept from then on (a
+//     push or pop compares its whole path at once, one LDS round trip).
+// Many hits at once are bounded by the issue of vector instructions: on 143,000 hits of
+// random hulls 4,235 per hit (5,146 with a heap from the first face on and the first
+// tetrahedron built by every lane), 1.35 ms (2.08).
 // The solver's uniform values come from v_readlane and ballots, so its branches are
 // scalar. Capacity is 64 K faces; running out of it returns 3, as does a plane distance
 // that is not finite (the heap's order then depends on the order of its comparisons):
@@ -64,6 +70,19 @@ __device__ __forceinline__ double half_max(double x)
     x = fmax(x, dpp64<0x114, 0xf>(x));
     x = fmax(x, dpp64<0x118, 0xf>(x));
     return fmax(x, dpp64<0x142, 0xa>(x));
+}
+
+// the minimum of all lanes, in every lane
+__device__ __forceinline__ double wave_min(double x)
+{
+    auto less = [](double a, double b) { return a < b ? a : b; };
+    x = less(dpp64<0x111, 0xf>(x), x);
+    x = less(dpp64<0x112, 0xf>(x), x);
+    x = less(dpp64<0x114, 0xf>(x), x);
+    x = less(dpp64<0x118, 0xf>(x), x);
+    x = less(dpp64<0x142, 0xa>(x), x);
+    x = less(dpp64<0x143, 0xc>(x), x);
+    return rl64(x, 63);
 }
 
 // The shape of this lane's half of the wavefront (A below lane 32, B above). A mesh of at
@@ -302,6 +321,10 @@ template <int K> struct solver
     uint64_t live[K]; // faces not obsolete (uniform)
     int npoly = 0, nfaces = 0, nheap = 0;
     uint32_t lane;
+    // without a heap until two live faces are nearest at once; lane i holds expansion i's
+    // face and (from bit 16) the face count after it, from which the heap can be built
+    bool heaped = false;
+    uint32_t hist = 0;
 
     __device__ explicit solver(store<K> &s) : m(s), lane(__lane_id())
     {
@@ -330,10 +353,7 @@ template <int K> struct solver
         uint32_t r = rl32(a[0], f & 63);
 #pragma unroll
         for (int k = 1; k < K; ++k)
-        {
-            const uint32_t t = rl32(a[k], f & 63);
-            r = sel((f >> 6) == k, t, r);
-        }
+            if (64 * k <= f) r = rl32(a[k], f & 63);
         return r;
     }
     __device__ __forceinline__ double real(const double (&a)[K], int f) const
@@ -341,23 +361,21 @@ template <int K> struct solver
         double r = rl64(a[0], f & 63);
 #pragma unroll
         for (int k = 1; k < K; ++k)
-        {
-            const double t = rl64(a[k], f & 63);
-            r = sel((f >> 6) == k, t, r);
-        }
+            if (64 * k <= f) r = rl64(a[k], f & 63);
         return r;
     }
-    __device__ __forceinline__ static bool bit(const uint64_t (&s)[K], uint32_t f)
+    // of faces 0 .. 64 N
+    template <int N> __device__ __forceinline__ static bool bit(const uint64_t (&s)[K], uint32_t f)
     {
         uint64_t w = s[0];
 #pragma unroll
-        for (int k = 1; k < K; ++k) w = sel((f >> 6) == static_cast<uint32_t>(k), s[k], w);
+        for (int k = 1; k < N; ++k) w = sel((f >> 6) == static_cast<uint32_t>(k), s[k], w);
         return (w >> (f & 63u)) & 1u;
     }
-    __device__ __forceinline__ static void clear(uint64_t (&s)[K], uint32_t f)
+    template <int N> __device__ __forceinline__ static void clear(uint64_t (&s)[K], uint32_t f)
     {
 #pragma unroll
-        for (int k = 0; k < K; ++k) s[k] &= ~((f >> 6) == static_cast<uint32_t>(k) ? 1ull << (f & 63u) : 0ull);
+        for (int k = 0; k < N; ++k) s[k] &= ~(N == 1 || (f >> 6) == static_cast<uint32_t>(k) ? 1ull << (f & 63u) : 0ull);
     }
 
     // push_heap's sift (libstdc++): the keys do not increase towards the root, so the
@@ -384,11 +402,12 @@ template <int K> struct solver
         }
         lds_sync();
     }
-    // pop_heap, and the faces it skips: the hole runs from the root to a leaf along the
+    // pop_heap, and the faces it skips (those before face `want`, or before the first live
+    // one where that is negative): the hole runs from the root to a leaf along the
     // smaller children (the right one of equal ones), then the last element rises from
     // that leaf past the keys above its own. The path is a run of bits; of its keys, the
     // ones not above the last element's move up by one node.
-    __device__ __forceinline__ int pop()
+    __device__ __forceinline__ int pop(int want)
     {
         while (nheap > 0)
         {
@@ -445,89 +464,114 @@ template <int K> struct solver
                 lds_sync();
             }
             --nheap;
-            if (bit(live, static_cast<uint32_t>(top))) return top;
+            if (want < 0 ? bit<K>(live, static_cast<uint32_t>(top)) : top == want) return top;
         }
         return -1;
     }
+    __device__ __forceinline__ void push_range(int from, int to)
+    {
+        for (int f = from; f < to; ++f) push(f, real(fd, f));
+    }
+    // The face that the heap's next pop returns (-1: none), for expansion it. That is the
+    // nearest live face, which the registers tell. Only where several are equally near does
+    // the order of the heap's operations so far decide: it is built then, by repeating them.
+    __device__ __forceinline__ int nearest(int it)
+    {
+        if (!heaped)
+        {
+            double b = __builtin_inf();
+#pragma unroll
+            for (int k = 0; k < K; ++k)
+                if (64 * k < nfaces)
+                {
+                    const double d = __builtin_amdgcn_inverse_ballot_w64(live[k]) ? fd[k] : __builtin_inf();
+                    b = d < b ? d : b;
+                }
+            b = wave_min(b);
+            int n = 0, f = -1;
+#pragma unroll
+            for (int k = 0; k < K; ++k)
+                if (64 * k < nfaces)
+                {
+                    const uint64_t eq = __ballot(fd[k] == b) & live[k];
+                    n += __popcll(eq);
+                    f = eq ? 64 * k + lowest_bit(eq) : f;
+                }
+            if (n < 2) return f;
+            heaped = true;
+            push_range(0, 4);
+            for (int i = 0, from = 4; i < it; ++i)
+            {
+                const uint32_t h = rl32(hist, i);
+                pop(static_cast<int>(h & 0xFFFFu));
+                push_range(from, static_cast<int>(h >> 16));
+                from = static_cast<int>(h >> 16);
+            }
+        }
+        return pop(-1);
+    }
 
-    // :355-388 from the four points; false when a plane distance is not finite
+    // :355-388 from the four points, face f in lane f; false when a plane distance is not
+    // finite. Faces (0 1 2), (0 2 3), (0 3 1), (1 3 2) run opposite ways along the edge that
+    // any two share, and still do if both are turned: a face's neighbour across an edge is the
+    // one without its third vertex, if it was turned alike.
     __device__ __forceinline__ bool initial_tetrahedron(const v3 (&q)[4])
     {
-        const int def[4][4] = {{0, 1, 2, 3}, {0, 2, 3, 1}, {0, 3, 1, 2}, {1, 3, 2, 0}};
-        int v[4][3], adj[4][3];
-        bool finite = true;
-#pragma unroll
-        for (int f = 0; f < 4; ++f)
+        const uint32_t f = lane & 3u;
+        const uint32_t i0 = f >> 1 & f, i1 = f == 0u ? 1u : (f == 1u ? 2u : 3u);
+        uint32_t i2 = f == 0u ? 2u : (f == 1u ? 3u : (f == 2u ? 1u : 2u)), iv = i1;
+        const uint32_t io = f == 0u ? 3u : (f == 3u ? 0u : f); // the vertex that face f lacks
+        auto at = [&](uint32_t i) { return sel3(i < 2u, sel3(i == 0u, q[0], q[1]), sel3(i == 2u, q[2], q[3])); };
+        const v3 pi = at(i0);
+        v3 nrm = cross(at(iv) - pi, at(i2) - pi);
+        if (sqn(nrm) < 1e-12)
+            nrm = mk(0.0, 0.0, 0.0);
+        else
+            nrm = normalized(nrm);
+        const bool turn = dot(nrm, at(io) - pi) > 0.0;
+        if (turn)
         {
-            const int i = def[f][0];
-            int v1 = def[f][1], v2 = def[f][2];
-            const v3 pi = q[i];
-            v3 nrm = cross(q[v1] - pi, q[v2] - pi);
-            if (sqn(nrm) < 1e-12)
-                nrm = mk(0.0, 0.0, 0.0);
-            else
-                nrm = normalized(nrm);
-            if (dot(nrm, q[def[f][3]] - pi) > 0.0)
-            {
-                const int t = v1;
-                v1 = v2;
-                v2 = t;
-                nrm = -nrm;
-            }
-            v[f][0] = i;
-            v[f][1] = v1;
-            v[f][2] = v2;
-            const double d = dot(nrm, pi);
-            finite = finite && isfinite(d);
-            const bool own = lane == static_cast<uint32_t>(f);
-            nx[0] = sel(own, nrm.x, nx[0]);
-            ny[0] = sel(own, nrm.y, ny[0]);
-            nz[0] = sel(own, nrm.z, nz[0]);
-            fd[0] = sel(own, d, fd[0]);
-            push(f, d);
+            const uint32_t t = iv;
+            iv = i2;
+            i2 = t;
+            nrm = -nrm;
         }
-#pragma unroll
-        for (int f = 0; f < 4; ++f) adj[f][0] = adj[f][1] = adj[f][2] = static_cast<int>(kNoFace);
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int j = i + 1; j < 4; ++j)
-#pragma unroll
-                for (int e1 = 0; e1 < 3; ++e1)
-#pragma unroll
-                    for (int e2 = 0; e2 < 3; ++e2)
-                        if (v[i][e1] == v[j][(e2 + 1) % 3] && v[i][(e1 + 1) % 3] == v[j][e2])
-                        {
-                            adj[i][e1] = j;
-                            adj[j][e2] = i;
-                        }
-#pragma unroll
-        for (int f = 0; f < 4; ++f)
+        const double d = dot(nrm, pi);
+        const uint32_t turned = static_cast<uint32_t>(__ballot(turn)) & 0xFu;
+        auto across = [&](uint32_t third)
         {
-            const bool own = lane == static_cast<uint32_t>(f);
-            fv[0] = sel(own, static_cast<uint32_t>(v[f][0] | v[f][1] << 8 | v[f][2] << 16), fv[0]);
-            f01[0] = sel(own, static_cast<uint32_t>(adj[f][0] | adj[f][1] << 16), f01[0]);
-            f2[0] = sel(own, static_cast<uint32_t>(adj[f][2]), f2[0]);
+            const uint32_t j = third == 0u ? 3u : (third == 3u ? 0u : third);
+            return ((turned >> j ^ turned >> f) & 1u) ? kNoFace : j;
+        };
+        if (lane < 4u)
+        {
+            nx[0] = nrm.x;
+            ny[0] = nrm.y;
+            nz[0] = nrm.z;
+            fd[0] = d;
+            fv[0] = i0 | iv << 8 | i2 << 16;
+            f01[0] = across(i2) | across(i0) << 16;
+            f2[0] = across(iv);
         }
         nfaces = 4;
         live[0] = 0xFull;
-        return finite;
+        return !__ballot(!isfinite(d));
     }
 
     // :315-353 from face f0 and the new point p. Horizon edge h (start, end, face across:
     // 8 + 8 + 16 bits) ends in lane (nfaces + h) & 63 of edges, the lane that will hold the
     // face built on it. Returns the edge count, -1 past 64 edges or stack entries.
-    __device__ __forceinline__ int silhouette(int f0, v3 p, uint32_t &edges)
+    template <int N> __device__ __forceinline__ int silhouette(int f0, v3 p, uint32_t &edges)
     {
         uint64_t vis[K];
 #pragma unroll
-        for (int k = 0; k < K; ++k)
+        for (int k = 0; k < N; ++k)
         {
             uint64_t seen = 0;
             if (64 * k < nfaces) seen = __ballot(dot(mk(nx[k], ny[k], nz[k]), p) > fd[k] + 1e-6);
             vis[k] = seen;
         }
-        clear(live, static_cast<uint32_t>(f0));
+        clear<N>(live, static_cast<uint32_t>(f0));
         uint32_t stack = 0; // entry i in lane i
         int sp = 0, nh = 0, cur = f0;
         for (;;)
@@ -537,10 +581,10 @@ template <int K> struct solver
             for (int i = 0; i < 3; ++i)
             {
                 const uint32_t nb = i == 0 ? (a01 & 0xFFFFu) : (i == 1 ? a01 >> 16 : a2);
-                if (nb == kNoFace || !bit(live, nb)) continue;
-                if (bit(vis, nb))
+                if (nb == kNoFace || !bit<N>(live, nb)) continue;
+                if (bit<N>(vis, nb))
                 {
-                    clear(live, nb);
+                    clear<N>(live, nb);
                     if (sp >= 64) return -1;
                     stack = lane == static_cast<uint32_t>(sp) ? nb : stack;
                     ++sp;
@@ -606,10 +650,11 @@ __device__ __forceinline__ int epa_solve(const shape &w, simplex &x, store<K> &s
     lds_sync();
     const v3 q[4] = {x.s0.p, x.s1.p, x.s2.p, x.s3.p};
     if (!e.initial_tetrahedron(q)) return 3;
-    for (int it = 0; it < 64; ++it)
+    int it = 0;
+    for (; it < 64; ++it)
     {
-        const int mf = e.pop();
-        if (mf < 0) break;
+        const int mf = e.nearest(it);
+        if (mf < 0) return 0;
         const v3 nrm = mk(e.real(e.nx, mf), e.real(e.ny, mf), e.real(e.nz, mf));
         const double d = e.real(e.fd, mf);
         const spt p = support<UV, MESH>(w, nrm);
@@ -620,9 +665,14 @@ __device__ __forceinline__ int epa_solve(const shape &w, simplex &x, store<K> &s
             return 1;
         }
         uint32_t edges = 0;
-        const int nh = e.silhouette(mf, p.p, edges);
+        const int nh = e.nfaces <= 64 ? e.template silhouette<1>(mf, p.p, edges) : e.template silhouette<K>(mf, p.p, edges);
         if (nh < 0) return 3;
-        if (nh == 0) break;
+        e.hist = e.lane == static_cast<uint32_t>(it) ? static_cast<uint32_t>(mf | (e.nfaces + nh) << 16) : e.hist;
+        if (nh == 0)
+        {
+            ++it;
+            break;
+        }
         const int base = e.nfaces;
         if (e.npoly >= store<K>::pcap || base + nh > store<K>::fcap) return 3;
         const int pi = e.npoly++;
@@ -660,6 +710,7 @@ __device__ __forceinline__ int epa_solve(const shape &w, simplex &x, store<K> &s
 #pragma unroll
             for (int k = 0; k < K; ++k)
             {
+                if (64 * k >= base) break;
                 const bool own = e.lane + 64u * k == across;
                 const bool at0 = (e.fv[k] & 0xFFu) == e_y, at1 = ((e.fv[k] >> 8) & 0xFFu) == e_y;
                 const uint32_t n01 = sel(at0, (e.f01[k] & 0xFFFF0000u) | fy,
@@ -672,6 +723,7 @@ __device__ __forceinline__ int epa_solve(const shape &w, simplex &x, store<K> &s
 #pragma unroll
         for (int k = 0; k < K; ++k)
         {
+            if (64 * k >= base + nh || 64 * k + 64 <= base) continue;
             const bool put = mine && slot == k;
             e.nx[k] = sel(put, fn.x, e.nx[k]);
             e.ny[k] = sel(put, fn.y, e.ny[k]);
@@ -688,10 +740,10 @@ __device__ __forceinline__ int epa_solve(const shape &w, simplex &x, store<K> &s
             const int lo = base > 64 * k ? base - 64 * k : 0, hi = end - 64 * k < 64 ? end - 64 * k : 64;
             e.live[k] |= lo < hi ? (~0ull >> (64 - hi)) & (~0ull << lo) : 0ull;
         }
-        for (int y = 0; y < nh; ++y) e.push(base + y, rl64(dist, (base + y) & 63));
+        if (e.heaped) e.push_range(base, end);
         e.nfaces = end;
     }
-    const int mf = e.pop();
+    const int mf = e.nearest(it);
     if (mf < 0) return 0;
     e.barycentric(mf, w, out);
     return 1;
