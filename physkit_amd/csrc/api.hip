@@ -1673,9 +1673,12 @@ void check_hit_total(pkg_ctx *ctx, uint32_t nq)
     if (sum > 0xFFFFFFFFull) throw pk_error(PKG_OVERFLOW_PAIRS, "query hit count exceeds 32-bit indexing");
 }
 
-void check_tree_walk(pkg_ctx *ctx)
+// returns the hits of the query with the most, where those were counted
+uint32_t check_tree_walk(pkg_ctx *ctx)
 {
-    if (ctx->read_counter(C_TREE_FAIL)) throw pk_error(PKG_DEVICE_ERROR, "query tree walk exceeded its node count");
+    ctx->read_counters(C_TREE_FAIL, C_QLONG);
+    if (ctx->h_counters[C_TREE_FAIL]) throw pk_error(PKG_DEVICE_ERROR, "query tree walk exceeded its node count");
+    return static_cast<uint32_t>(ctx->h_counters[C_QLONG]);
 }
 } // namespace
 
@@ -1699,12 +1702,13 @@ pkg_status pkg_raycast(pkg_ctx *ctx, uint32_t n_rays, const double *origins, con
         lbvh_dev t = ctx->query_tree();
         bodies_dev b = ctx->B();
         unsigned long long *fail = ctx->counters.p + C_TREE_FAIL;
-        ctx->reset_counter(C_TREE_FAIL);
+        launch_fill_u64(ctx->counters.p + C_TREE_FAIL, 0ull, 2, st); // and C_QLONG
         ctx->q_cnt.reserve(n_rays);
         launch_ray_count(t, b, n_rays, ctx->q_org.p, ctx->q_dir.p, ctx->q_maxd.p, rw, ctx->q_cnt.p, fail, st);
         check_hit_total(ctx, n_rays);
+        launch_longest(ctx->q_cnt.p, n_rays, ctx->counters.p + C_QLONG, st);
         const uint32_t m = ctx->scan_counts(n_rays);
-        check_tree_walk(ctx);
+        const uint32_t longest = check_tree_walk(ctx);
         hip_check(hipMemcpyAsync(offsets, ctx->q_off.p, (static_cast<size_t>(n_rays) + 1) * sizeof(uint32_t),
                                  hipMemcpyDeviceToHost, st),
                   "offsets");
@@ -1713,11 +1717,11 @@ pkg_status pkg_raycast(pkg_ctx *ctx, uint32_t n_rays, const double *origins, con
         if (!m || cap < m) return PKG_OK;
         if (!ids || !dists) throw pk_error(PKG_INVALID_ARG, "ids and dists are needed when cap >= total");
         query_scratch qs = ctx->qscratch(m);
-        launch_ray_fill(t, b, n_rays, ctx->q_org.p, ctx->q_dir.p, ctx->q_maxd.p, rw, ctx->q_off.p, qs.hid, qs.hd,
-                        qs.hq, fail, st);
+        launch_ray_fill(t, b, n_rays, ctx->q_org.p, ctx->q_dir.p, ctx->q_maxd.p, rw, ctx->q_cnt.p, ctx->q_off.p, qs.hid,
+                        qs.hd, qs.hq, fail, st);
         ctx->q_out_id.reserve(m);
         ctx->q_out_d.reserve(m);
-        launch_hits_sort(qs, m, ctx->n, n_rays, true, ctx->q_out_id.p, ctx->q_out_d.p, ctx->sc, st);
+        launch_hits_sort(qs, m, ctx->n, n_rays, longest, ctx->q_off.p, true, ctx->q_out_id.p, ctx->q_out_d.p, ctx->sc, st);
         hip_check(hipMemcpyAsync(ids, ctx->q_out_id.p, m * sizeof(uint32_t), hipMemcpyDeviceToHost, st), "ids");
         hip_check(hipMemcpyAsync(dists, ctx->q_out_d.p, m * sizeof(double), hipMemcpyDeviceToHost, st), "dists");
         hip_check(hipStreamSynchronize(st), "stream sync");
@@ -1801,12 +1805,13 @@ pkg_status pkg_query_aabb(pkg_ctx *ctx, uint32_t n_boxes, const double *boxes, c
         lbvh_dev t = ctx->query_tree();
         bodies_dev b = ctx->B();
         unsigned long long *fail = ctx->counters.p + C_TREE_FAIL;
-        ctx->reset_counter(C_TREE_FAIL);
+        launch_fill_u64(ctx->counters.p + C_TREE_FAIL, 0ull, 2, st); // and C_QLONG
         ctx->q_cnt.reserve(n_boxes);
         launch_box_count(t, b, n_boxes, ctx->q_box.p, qw, ctx->q_cnt.p, fail, st);
         check_hit_total(ctx, n_boxes);
+        launch_longest(ctx->q_cnt.p, n_boxes, ctx->counters.p + C_QLONG, st);
         const uint32_t m = ctx->scan_counts(n_boxes);
-        check_tree_walk(ctx);
+        const uint32_t longest = check_tree_walk(ctx);
         hip_check(hipMemcpyAsync(offsets, ctx->q_off.p, (static_cast<size_t>(n_boxes) + 1) * sizeof(uint32_t),
                                  hipMemcpyDeviceToHost, st),
                   "offsets");
@@ -1815,9 +1820,9 @@ pkg_status pkg_query_aabb(pkg_ctx *ctx, uint32_t n_boxes, const double *boxes, c
         if (!m || cap < m) return PKG_OK;
         if (!ids) throw pk_error(PKG_INVALID_ARG, "ids are needed when cap >= total");
         query_scratch qs = ctx->qscratch(m);
-        launch_box_fill(t, b, n_boxes, ctx->q_box.p, qw, ctx->q_off.p, qs.hid, qs.hq, fail, st);
+        launch_box_fill(t, b, n_boxes, ctx->q_box.p, qw, ctx->q_cnt.p, ctx->q_off.p, qs.hid, qs.hq, fail, st);
         ctx->q_out_id.reserve(m);
-        launch_hits_sort(qs, m, ctx->n, n_boxes, false, ctx->q_out_id.p, nullptr, ctx->sc, st);
+        launch_hits_sort(qs, m, ctx->n, n_boxes, longest, ctx->q_off.p, false, ctx->q_out_id.p, nullptr, ctx->sc, st);
         hip_check(hipMemcpyAsync(ids, ctx->q_out_id.p, m * sizeof(uint32_t), hipMemcpyDeviceToHost, st), "ids");
         hip_check(hipStreamSynchronize(st), "stream sync");
         check_tree_walk(ctx);

@@ -16,6 +16,18 @@ namespace pk
 namespace
 {
 constexpr int kBlock = 256;
+// Up to this many rays or boxes kSlices threads share one; beyond, the chip is full without and
+// the slices' first steps only add work. Whole calls over 32,768 bodies with 1, 16 and 32
+// slices: 1,024 rays 1.23, 0.97 and 0.81 ms, 16,384 rays 1.51, 1.26 and 1.19, 65,536 rays
+// 2.09, 2.27 and 2.66; 4,096 boxes 1.53, 1.31 and 1.22, 16,384 boxes 1.74, 1.95 and 1.89.
+constexpr uint32_t kSliceRays = 16384;
+constexpr uint32_t kSliceBoxes = 8192;
+constexpr uint32_t kSlices = 32;
+// Up to this many hits a query, its hits are sorted by counting; above, by radix passes over all
+// hits (12 of them for rays). 33,500 hits of 1,024 boxes, at most 159 each: 1.06 ms for the whole
+// call against 1.15; 915,000 of 8,192, at most 442: 2.92 against 3.05. The work grows with
+// the square.
+constexpr uint32_t kRankMax = 512;
 unsigned grid(size_t n) { return static_cast<unsigned>((n + kBlock - 1) / kBlock); }
 
 // ray::intersect_distance: slab test with NaN products (0 * inf) replaced by the
@@ -92,17 +104,33 @@ __device__ __forceinline__ qray load_ray(const lbvh_dev &t, uint32_t r, const do
 __device__ __forceinline__ bool node_in_range(const lbvh_dev &t, uint32_t node, uint32_t wlo, uint32_t whi)
 { return t.first[node] <= whi && (t.lastf[node] & 0x7fffffffu) >= wlo; }
 
-// Calls leaf(body, distance) for every live leaf of the range the ray meets within
-// max(); max() may shrink as leaves are accepted (closest-hit pruning).
-template <class Leaf, class Max>
-__device__ __forceinline__ void walk_ray(const lbvh_dev &t, const bodies_dev &b, const qray &q, Leaf &&leaf,
-                                         Max &&maxd, unsigned long long *fail)
+// The walks that list every hit are chains of dependent node loads, the longest of a few
+// hundred: with few queries there are too few threads to hide them, and kSlices threads
+// share one, each walking its slice of the leaves (from its first leaf through the escape links,
+// a rejected node skipping past its last leaf, up to the next slice's first).
+struct qslice
+{
+    uint32_t at, end; // the first leaf below the walk's node, the slice's end
+    __device__ __forceinline__ qslice(uint32_t wlo, uint32_t whi, uint32_t s)
+    {
+        const uint64_t len = static_cast<uint64_t>(whi) - wlo + 1;
+        at = wlo + static_cast<uint32_t>(len * s / kSlices);
+        end = wlo + static_cast<uint32_t>(len * (s + 1) / kSlices);
+    }
+};
+
+// Calls leaf(body, distance) for every live leaf of the range (SLICED: of its slice s) that
+// the ray meets.
+template <bool SLICED, class Leaf>
+__device__ __forceinline__ void walk_ray(const lbvh_dev &t, const bodies_dev &b, const qray &q, uint32_t s, Leaf &&leaf,
+                                         unsigned long long *fail)
 {
     const uint32_t n = t.n;
     if (n == 0 || q.whi < q.wlo || q.whi == 0xFFFFFFFFu) return;
     const bool ranged = q.wlo != 0 || q.whi != n - 1;
-    uint32_t node = 0;
-    for (uint32_t guard = 0; node != kNone; ++guard)
+    qslice sl(q.wlo, q.whi, s);
+    uint32_t node = SLICED ? n - 1 + sl.at : 0u;
+    for (uint32_t guard = 0; node != kNone && (!SLICED || sl.at < sl.end); ++guard)
     {
         if (guard >= 2 * n)
         {
@@ -114,22 +142,27 @@ __device__ __forceinline__ void walk_ray(const lbvh_dev &t, const bodies_dev &b,
         {
             float4 lo = t.inode_lo[node], hi = t.inode_hi[node];
             next = __float_as_uint(hi.w);
+            const uint32_t past = SLICED ? (t.lastf[node] & 0x7fffffffu) + 1u : 0u;
             double td;
-            bool hit = ray_slab(q.o, q.inv, mk(lo.x, lo.y, lo.z), mk(hi.x, hi.y, hi.z), maxd(), td);
-            if (hit && ranged) hit = node_in_range(t, node, q.wlo, q.whi);
-            if (hit) next = __float_as_uint(lo.w);
+            bool hit = ray_slab(q.o, q.inv, mk(lo.x, lo.y, lo.z), mk(hi.x, hi.y, hi.z), q.maxd, td);
+            if (!SLICED && hit && ranged) hit = node_in_range(t, node, q.wlo, q.whi);
+            if (hit)
+                next = __float_as_uint(lo.w);
+            else
+                sl.at = past;
         }
         else
         {
             const uint32_t j = node - (n - 1);
             next = n == 1 ? kNone : t.escape[node];
+            sl.at = j + 1;
             if (j >= q.wlo && j <= q.whi)
             {
                 const uint32_t body = t.leaf_body[j];
                 const double *p = t.leaf_box + static_cast<size_t>(j) * 6;
                 double td;
                 if (b.is_static[body] != 2 &&
-                    ray_slab(q.o, q.inv, mk(p[0], p[1], p[2]), mk(p[3], p[4], p[5]), maxd(), td))
+                    ray_slab(q.o, q.inv, mk(p[0], p[1], p[2]), mk(p[3], p[4], p[5]), q.maxd, td))
                     leaf(body, td);
             }
         }
@@ -261,45 +294,68 @@ __global__ void __launch_bounds__(kBlock)
     out_d[r] = best_id == kNone ? __builtin_inf() : best;
 }
 
-// every hit: FILL = false counts per ray, FILL = true writes (body, distance, ray) at
-// the ray's offset in walk order
-template <bool FILL>
+// Writes the hits of query r into its slots [off[r], off[r + 1]), never past them: in walk order,
+// or (SLICED) from the last down, the count that is left telling the place. (Hits buffered
+// sixteen at a time took the same: 4,096 rays 0.97 ms against 0.92, 1,024 boxes 1.01 against
+// 1.05.)
+template <bool SLICED> struct hit_writer
+{
+    uint32_t r, beg, end, k;
+    uint32_t *cnt, *hid, *hq;
+    double *hd;
+
+    __device__ __forceinline__ void add(uint32_t body, double dist)
+    {
+        const uint32_t at = SLICED ? atomicSub(&cnt[r], 1u) - 1u : k++;
+        if (at >= end - beg) return;
+        hid[beg + at] = body;
+        hq[beg + at] = r;
+        if (hd) hd[beg + at] = dist;
+    }
+};
+
+// the hits of a query's thread (SLICED: counts start at 0)
+template <bool SLICED> __device__ __forceinline__ void add_count(uint32_t *cnt, uint32_t r, uint32_t k)
+{
+    if (!SLICED)
+        cnt[r] = k;
+    else if (k)
+        atomicAdd(&cnt[r], k);
+}
+
+// every hit: FILL = false counts per ray, FILL = true writes (body, distance, ray) into
+// the ray's slots.
+template <bool FILL, bool SLICED>
 __global__ void __launch_bounds__(kBlock)
     k_ray_all(lbvh_dev t, bodies_dev b, uint32_t nr, const double *org, const double *dir, const double *maxd,
               const uint32_t *rw, uint32_t *cnt, const uint32_t *off, uint32_t *hid, double *hd, uint32_t *hq,
               unsigned long long *fail)
 {
-    uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x, r = SLICED ? i / kSlices : i;
     if (r >= nr) return;
     const qray q = load_ray(t, r, org, dir, maxd, rw);
-    uint32_t k = FILL ? off[r] : 0u;
-    const uint32_t end = FILL ? off[r + 1] : 0u;
-    walk_ray(
-        t, b, q,
+    uint32_t k = 0;
+    hit_writer<SLICED> w{r, FILL ? off[r] : 0u, FILL ? off[r + 1] : 0u, 0u, cnt, hid, hq, hd};
+    walk_ray<SLICED>(
+        t, b, q, i % kSlices,
         [&](uint32_t body, double d)
         {
             if (FILL)
-            {
-                if (k < end) // the fill walk repeats the counting walk; never past the ray's slots
-                {
-                    hid[k] = body;
-                    hd[k] = d;
-                    hq[k] = r;
-                }
-            }
-            ++k;
+                w.add(body, d);
+            else
+                ++k;
         },
-        [&]() { return q.maxd; }, fail);
-    if (!FILL) cnt[r] = k;
+        fail);
+    if (!FILL) add_count<SLICED>(cnt, r, k);
 }
 
 // AABB query: leaves whose tree bounds intersect the box (bounds.h:87-92)
-template <bool FILL>
+template <bool FILL, bool SLICED>
 __global__ void __launch_bounds__(kBlock)
     k_box_all(lbvh_dev t, bodies_dev b, uint32_t nq, const double *boxes, const uint32_t *qw, uint32_t *cnt,
               const uint32_t *off, uint32_t *hid, uint32_t *hq, unsigned long long *fail)
 {
-    uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x, r = SLICED ? i / kSlices : i;
     if (r >= nq) return;
     const uint32_t n = t.n;
     box3 q;
@@ -330,11 +386,13 @@ __global__ void __launch_bounds__(kBlock)
             whi = 0;
         }
     }
-    uint32_t k = FILL ? off[r] : 0u;
-    const uint32_t end = FILL ? off[r + 1] : 0u;
+    uint32_t k = 0;
+    hit_writer<SLICED> w{r, FILL ? off[r] : 0u, FILL ? off[r + 1] : 0u, 0u, cnt, hid, hq, nullptr};
     const bool ranged = wlo != 0 || whi != n - 1;
-    uint32_t node = (n == 0 || whi < wlo || whi == 0xFFFFFFFFu) ? kNone : 0u;
-    for (uint32_t guard = 0; node != kNone; ++guard)
+    const bool none = n == 0 || whi < wlo || whi == 0xFFFFFFFFu;
+    qslice sl(wlo, whi, i % kSlices);
+    uint32_t node = none ? kNone : (SLICED ? n - 1 + sl.at : 0u);
+    for (uint32_t guard = 0; node != kNone && (!SLICED || sl.at < sl.end); ++guard)
     {
         if (guard >= 2 * n)
         {
@@ -347,13 +405,16 @@ __global__ void __launch_bounds__(kBlock)
             float4 lo = t.inode_lo[node], hi = t.inode_hi[node];
             bool ov = lo.x <= qhi[0] && hi.x >= qlo[0] && lo.y <= qhi[1] && hi.y >= qlo[1] && lo.z <= qhi[2] &&
                       hi.z >= qlo[2];
-            if (ov && ranged) ov = node_in_range(t, node, wlo, whi);
+            const uint32_t past = SLICED ? (t.lastf[node] & 0x7fffffffu) + 1u : 0u;
+            if (!SLICED && ov && ranged) ov = node_in_range(t, node, wlo, whi);
             next = __float_as_uint(ov ? lo.w : hi.w);
+            if (!ov) sl.at = past;
         }
         else
         {
             const uint32_t j = node - (n - 1);
             next = n == 1 ? kNone : t.escape[node];
+            sl.at = j + 1;
             if (j >= wlo && j <= whi)
             {
                 const uint32_t body = t.leaf_body[j];
@@ -363,18 +424,16 @@ __global__ void __launch_bounds__(kBlock)
                 lb.max = mk(p[3], p[4], p[5]);
                 if (b.is_static[body] != 2 && box_intersects(lb, q))
                 {
-                    if (FILL && k < end)
-                    {
-                        hid[k] = body;
-                        hq[k] = r;
-                    }
-                    ++k;
+                    if (FILL)
+                        w.add(body, 0.0);
+                    else
+                        ++k;
                 }
             }
         }
         node = next;
     }
-    if (!FILL) cnt[r] = k;
+    if (!FILL) add_count<SLICED>(cnt, r, k);
 }
 
 // sort keys: u32 or the bits of a non-negative double (monotone as unsigned integers),
@@ -402,6 +461,38 @@ __global__ void k_gather_hits(const uint32_t *perm, uint32_t n, const uint32_t *
     uint32_t s = perm[i];
     out_id[i] = hid[s];
     if (hd) out_d[i] = hd[s];
+}
+
+__global__ void k_longest(const uint32_t *cnt, uint32_t n, unsigned long long *longest)
+{
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    block_max(longest, i < n ? cnt[i] : 0u);
+}
+
+// Hits sorted inside their queries' slots: a thread per hit counts the query's hits that come
+// before it, by (distance, body) or body. A body is a query's hit at most once.
+template <bool DIST>
+__global__ void __launch_bounds__(kBlock)
+    k_rank_hits(uint32_t m, const uint32_t *off, const uint32_t *hid, const double *hd, const uint32_t *hq, uint32_t *out_id,
+                double *out_d)
+{
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= m) return;
+    const uint32_t beg = off[hq[i]], end = off[hq[i] + 1], id = hid[i];
+    const double d = DIST ? hd[i] : 0.0;
+    uint32_t rank = 0;
+    for (uint32_t j = beg; j < end; ++j)
+    {
+        bool before = hid[j] < id;
+        if (DIST)
+        {
+            const double o = hd[j];
+            before = o < d || (o == d && before);
+        }
+        rank += before ? 1u : 0u;
+    }
+    out_id[beg + rank] = id;
+    if (DIST) out_d[beg + rank] = d;
 }
 
 int bits_for(uint64_t maxv)
@@ -441,32 +532,66 @@ void launch_ray_closest(const lbvh_dev &t, const uint4 *rn, const bodies_dev &b,
 void launch_ray_count(const lbvh_dev &t, const bodies_dev &b, uint32_t nr, const double *org, const double *dir,
                       const double *maxd, const uint32_t *rw, uint32_t *cnt, unsigned long long *fail, hipStream_t st)
 {
-    if (nr)
-        k_ray_all<false><<<grid(nr), kBlock, 0, st>>>(t, b, nr, org, dir, maxd, rw, cnt, nullptr, nullptr, nullptr,
-                                                       nullptr, fail);
+    if (!nr) return;
+    if (nr <= kSliceRays)
+    {
+        launch_fill_u32(cnt, 0u, nr, st);
+        k_ray_all<false, true><<<grid(nr * kSlices), kBlock, 0, st>>>(t, b, nr, org, dir, maxd, rw, cnt, nullptr, nullptr,
+                                                                     nullptr, nullptr, fail);
+    }
+    else
+        k_ray_all<false, false><<<grid(nr), kBlock, 0, st>>>(t, b, nr, org, dir, maxd, rw, cnt, nullptr, nullptr, nullptr,
+                                                             nullptr, fail);
 }
 void launch_ray_fill(const lbvh_dev &t, const bodies_dev &b, uint32_t nr, const double *org, const double *dir,
-                     const double *maxd, const uint32_t *rw, const uint32_t *off, uint32_t *hid, double *hd,
+                     const double *maxd, const uint32_t *rw, uint32_t *cnt, const uint32_t *off, uint32_t *hid, double *hd,
                      uint32_t *hq, unsigned long long *fail, hipStream_t st)
 {
-    if (nr)
-        k_ray_all<true><<<grid(nr), kBlock, 0, st>>>(t, b, nr, org, dir, maxd, rw, nullptr, off, hid, hd, hq, fail);
+    if (!nr) return;
+    if (nr <= kSliceRays)
+        k_ray_all<true, true><<<grid(nr * kSlices), kBlock, 0, st>>>(t, b, nr, org, dir, maxd, rw, cnt, off, hid, hd, hq, fail);
+    else
+        k_ray_all<true, false><<<grid(nr), kBlock, 0, st>>>(t, b, nr, org, dir, maxd, rw, cnt, off, hid, hd, hq, fail);
 }
 void launch_box_count(const lbvh_dev &t, const bodies_dev &b, uint32_t nq, const double *boxes, const uint32_t *qw,
                       uint32_t *cnt, unsigned long long *fail, hipStream_t st)
 {
-    if (nq) k_box_all<false><<<grid(nq), kBlock, 0, st>>>(t, b, nq, boxes, qw, cnt, nullptr, nullptr, nullptr, fail);
+    if (!nq) return;
+    if (nq <= kSliceBoxes)
+    {
+        launch_fill_u32(cnt, 0u, nq, st);
+        k_box_all<false, true><<<grid(nq * kSlices), kBlock, 0, st>>>(t, b, nq, boxes, qw, cnt, nullptr, nullptr, nullptr, fail);
+    }
+    else
+        k_box_all<false, false><<<grid(nq), kBlock, 0, st>>>(t, b, nq, boxes, qw, cnt, nullptr, nullptr, nullptr, fail);
 }
 void launch_box_fill(const lbvh_dev &t, const bodies_dev &b, uint32_t nq, const double *boxes, const uint32_t *qw,
-                     const uint32_t *off, uint32_t *hid, uint32_t *hq, unsigned long long *fail, hipStream_t st)
+                     uint32_t *cnt, const uint32_t *off, uint32_t *hid, uint32_t *hq, unsigned long long *fail, hipStream_t st)
 {
-    if (nq) k_box_all<true><<<grid(nq), kBlock, 0, st>>>(t, b, nq, boxes, qw, nullptr, off, hid, hq, fail);
+    if (!nq) return;
+    if (nq <= kSliceBoxes)
+        k_box_all<true, true><<<grid(nq * kSlices), kBlock, 0, st>>>(t, b, nq, boxes, qw, cnt, off, hid, hq, fail);
+    else
+        k_box_all<true, false><<<grid(nq), kBlock, 0, st>>>(t, b, nq, boxes, qw, cnt, off, hid, hq, fail);
 }
 
-void launch_hits_sort(query_scratch &qs, uint32_t m, uint32_t n_bodies, uint32_t n_queries, bool by_distance,
-                      uint32_t *out_id, double *out_d, sort_scratch &sc, hipStream_t st)
+void launch_longest(const uint32_t *cnt, uint32_t n, unsigned long long *longest, hipStream_t st)
+{
+    if (n) k_longest<<<grid(n), kBlock, 0, st>>>(cnt, n, longest);
+}
+void launch_hits_sort(query_scratch &qs, uint32_t m, uint32_t n_bodies, uint32_t n_queries, uint32_t longest,
+                      const uint32_t *off, bool by_distance, uint32_t *out_id, double *out_d, sort_scratch &sc,
+                      hipStream_t st)
 {
     if (!m) return;
+    if (longest <= kRankMax)
+    {
+        if (by_distance)
+            k_rank_hits<true><<<grid(m), kBlock, 0, st>>>(m, off, qs.hid, qs.hd, qs.hq, out_id, out_d);
+        else
+            k_rank_hits<false><<<grid(m), kBlock, 0, st>>>(m, off, qs.hid, qs.hd, qs.hq, out_id, out_d);
+        return;
+    }
     // stable passes from the least significant criterion: body, then distance, then query
     k_key_u32<<<grid(m), kBlock, 0, st>>>(qs.hid, nullptr, m, qs.keys);
     k_iota<<<grid(m), kBlock, 0, st>>>(qs.perm, m);

@@ -88,7 +88,7 @@ enum counter_slot
     C_EPA_BIG_FAIL = 9,
     C_EVENTS = 10,
     C_TREE_FAIL = 11,
-    C_EPA_OVF2 = 12, // overflows of the 512-face store, rerun in global memory
+    C_QLONG = 12, // hits of the query with the most
     C_KEEP = 13,
     C_ISL_MAX = 14,
     C_NCOL = 15,
@@ -98,6 +98,7 @@ enum counter_slot
     C_MSLOTS = 19,    // manifold data slots taken by the manifold update
     C_MLIVE = 20,     // pairs listed for the manifold update (see launch_manifold_update)
     C_MLEAF = 21,     // leaves listed for the pair query (dynamic and moved)
+    C_EPA_OVF2 = 22,  // overflows of the 512-face store, rerun in global memory
     // pair query cursors: one per output region, each in its own 256-byte line, so
     // wavefronts reserving output space spread their atomics over kPairRegions
     // addresses instead of serialising on one
@@ -478,16 +479,20 @@ void launch_ray_closest(const lbvh_dev &t, const uint4 *rn, const bodies_dev &b,
 void launch_ray_count(const lbvh_dev &t, const bodies_dev &b, uint32_t nr, const double *org, const double *dir,
                       const double *maxd, const uint32_t *rw, uint32_t *cnt, unsigned long long *fail, hipStream_t st);
 void launch_ray_fill(const lbvh_dev &t, const bodies_dev &b, uint32_t nr, const double *org, const double *dir,
-                     const double *maxd, const uint32_t *rw, const uint32_t *off, uint32_t *hid, double *hd,
-                     uint32_t *hq, unsigned long long *fail, hipStream_t st);
+                     const double *maxd, const uint32_t *rw, uint32_t *cnt, const uint32_t *off, uint32_t *hid,
+                     double *hd, uint32_t *hq, unsigned long long *fail, hipStream_t st);
 void launch_box_count(const lbvh_dev &t, const bodies_dev &b, uint32_t nq, const double *boxes, const uint32_t *qw,
                       uint32_t *cnt, unsigned long long *fail, hipStream_t st);
 void launch_box_fill(const lbvh_dev &t, const bodies_dev &b, uint32_t nq, const double *boxes, const uint32_t *qw,
-                     const uint32_t *off, uint32_t *hid, uint32_t *hq, unsigned long long *fail, hipStream_t st);
+                     uint32_t *cnt, const uint32_t *off, uint32_t *hid, uint32_t *hq, unsigned long long *fail,
+                     hipStream_t st);
 // sorts the m hits by (query, distance, body) (by_distance) or (query, body) and writes
 // bodies (and distances) in that order
-void launch_hits_sort(query_scratch &qs, uint32_t m, uint32_t n_bodies, uint32_t n_queries, bool by_distance,
-                      uint32_t *out_id, double *out_d, sort_scratch &sc, hipStream_t st);
+void launch_hits_sort(query_scratch &qs, uint32_t m, uint32_t n_bodies, uint32_t n_queries, uint32_t longest,
+                      const uint32_t *off, bool by_distance, uint32_t *out_id, double *out_d, sort_scratch &sc,
+                      hipStream_t st);
+// the largest of cnt[0..n), into a counter that starts at 0
+void launch_longest(const uint32_t *cnt, uint32_t n, unsigned long long *longest, hipStream_t st);
 
 // ---------------- k_joint.hip ----------------
 // Joint records: kJW planes of `cap` doubles (word w of joint j at rec[w * cap + j]),
