@@ -198,11 +198,11 @@ def stage_bytes(s, c, pairs, hits_frac, pos, iterations, mixed, tree_refits=0, i
                         n if M == 0 and K == 0 else 48 * M + 80 * n + 36 * K + 20 * P),
         "gjk": ("GJK stage (k_gjk_cull" + (", k_gjk32" if mixed else "") + ", k_gjk)",
                 (algorithmic_bytes("gjk", s, pairs, hits_frac, pos) if len(pairs) else 0.0) + (6 * P if fused else 0)),
-        "epa": ("k_epa (+ larger-store reruns)", algorithmic_bytes("epa", s, pairs, hits_frac) if len(pairs) else 0.0),
+        "epa": ("k_epa_wave (+ larger-store reruns)", algorithmic_bytes("epa", s, pairs, hits_frac) if len(pairs) else 0.0),
         "manifold": ("k_manifold" if fused else "k_manifold_live, k_manifold",
                      (0 if fused else 8 * P) + 28 * c["gjk_listed"] + 208 * C + 192 * H),
         "solver": ("contact solver stage", 496 * R),
-        "solve_iterations": ("k_solve_islands" + ("<true> (FP32 rows)" if mixed else "<false>"), R * (38 * sr + 96)),
+        "solve_iterations": ("k_solve_chunks" + ("<true> (FP32 rows)" if mixed else "<false>"), R * (38 * sr + 96)),
         "integrate_pos": ("k_integrate_pos", (n + 448 * nd) / steps),
     }
     if not integrate:

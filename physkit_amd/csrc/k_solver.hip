@@ -808,12 +808,12 @@ __device__ __forceinline__ void solve_chunk_reg(const uint64_t *keys, const uint
             if (valid[q]) ctc_store_acc(k[q], r, static_cast<uint32_t>(q) * cap + t);
 }
 
-// kIslandThreads threads. A chunk of at most kIslandThreads manifolds is solved one
-// manifold per thread in registers, one of at most CAP manifolds with the velocities in
-// LDS and each manifold's rows read per pass, a larger one (an island of more than CAP
-// manifolds) from global memory. CAP 256 (every island at most 256 manifolds, windows
-// sized to match) halves the LDS, and its FP32 form is held to two waves per SIMD, so
-// two workgroups share a CU; CAP 512 keeps every register for its long islands.
+// For scenes whose longest island passes what one workgroup colours and keeps in registers
+// (k_island.hip, which takes 64 pyramids of 330 manifolds through a step in 0.95 ms; this
+// kernel with the global colouring and row setup before it 1.65). A chunk of at most
+// kIslandThreads manifolds is solved one manifold per thread in registers, one of at most
+// CAP manifolds with the velocities in LDS and each manifold's rows read per pass, a larger
+// one (an island of more than CAP manifolds) from global memory.
 constexpr int kIslandThreads = 256;
 constexpr int CAP = 2 * kIslandThreads;
 template <bool F32>
