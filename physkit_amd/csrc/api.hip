@@ -1300,7 +1300,7 @@ pkg_status pkg_create(pkg_ctx **out, const pkg_config *cfg)
         c->counters.reserve(C_NCOUNTERS);
         if (const char *e = std::getenv("PKG_PAIR_REGION_MIN_LEAVES"))
             c->region_min_leaves = static_cast<uint32_t>(std::strtoul(e, nullptr, 10));
-        c->scene.reserve(6);
+        c->scene.reserve(12);
     }
     catch (const pk_error &e)
     {

@@ -11,6 +11,7 @@
 // with the child and escape links); every leaf test uses the exact FP64 leaf box, so
 // each overlap decision is the reference's aabb::intersects.
 #include "pk_access.hpp"
+#include "pk_trim.hpp"
 
 namespace pk
 {
@@ -106,32 +107,27 @@ __global__ void __launch_bounds__(kBlock) k_scene_bounds(bodies_dev b, unsigned 
     }
 }
 
-// The Morton grid's range on one axis (workgroup k: axis k): the exact bounds cut back to
-// those of the bulk of the leaves, so that a few bodies far away (fallen off the ground,
-// flung off by an unstable contact) do not squeeze all others into a handful of cells, which
-// leaves the hierarchy without spatial order inside a world and lets every query walk most
-// of it. The bulk: 1,024 centroids spread over the body ids, sorted in LDS, without a 64th at
-// either end, widened by half its extent each way (a scene without such outliers keeps its
-// exact bounds). Leaves outside share the border cells; pairs and query answers do not
-// depend on the tree's shape. On 720,000 bodies of batched worlds whose fastest bodies had
-// left by far, the pair query took 10 ms on a step that moved every leaf and 3 ms on one that
-// moved 786; with the cut 0.6 and 0.4-0.8 ms, for about 12 us per full build.
-constexpr int kTrimSample = 1024;
+// The bulk of the leaves on one axis (workgroup k: axis k; pk_trim.hpp), for the Morton grid's
+// range: 1,024 centroids spread over the body ids (all of a smaller scene), sorted in LDS.
+// Pairs and query answers do not depend on the tree's shape. On 720,000 bodies of batched
+// worlds whose fastest bodies had left by far, the pair query took 10 ms on a step that
+// moved every leaf and 3 ms on one that moved 786; with the cut 0.6 and 0.4-0.8 ms, for about
+// 12 us per full build.
 __global__ void __launch_bounds__(kTrimSample) k_scene_trim(bodies_dev b, unsigned long long *scene)
 {
     __shared__ double v[kTrimSample];
     const uint32_t t = threadIdx.x, k = blockIdx.x;
     double x = __builtin_inf();
-    const bool spread = b.n > static_cast<uint32_t>(kTrimSample);
+    const bool spread = b.n > kTrimSample;
     if (spread || t < b.n)
     {
-        const size_t i = 6 * (spread ? static_cast<size_t>(t) * b.n / kTrimSample : t);
+        const size_t i = 6 * static_cast<size_t>(spread ? trim_sample(t, b.n) : t);
         const double c = (b.fat[i + k] + b.fat[i + k + 3]) * 0.5;
         if (isfinite(c)) x = c;
     }
     const int finite = __syncthreads_count(isfinite(x));
     v[t] = x;
-    for (uint32_t size = 2; size <= static_cast<uint32_t>(kTrimSample); size <<= 1) // bitonic sort, infinities last
+    for (uint32_t size = 2; size <= kTrimSample; size <<= 1) // bitonic sort, infinities last
         for (uint32_t stride = size >> 1; stride > 0; stride >>= 1)
         {
             __syncthreads();
@@ -147,11 +143,11 @@ __global__ void __launch_bounds__(kTrimSample) k_scene_trim(bodies_dev b, unsign
             }
         }
     __syncthreads();
-    if (t != 0 || finite == 0) return;
-    const double lo = v[finite / 64], hi = v[finite - 1 - finite / 64], half = (hi - lo) * 0.5;
-    const double l = fmax(unord(scene[k]), lo - half), h = fmin(unord(scene[3 + k]), hi + half);
-    scene[k] = ord(l);
-    scene[3 + k] = ord(h);
+    if (t != 0) return;
+    double lo = 0.0, hi = 0.0;
+    if (finite) trim_axis(v, finite, lo, hi);
+    scene[6 + 2 * k] = ord(lo);
+    scene[7 + 2 * k] = ord(hi);
 }
 
 __device__ __forceinline__ uint64_t split3(uint64_t x)
@@ -170,9 +166,12 @@ __global__ void k_morton(bodies_dev b, lbvh_dev t, const unsigned long long *sce
     uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= b.n) return;
     uint64_t q[3];
+    double widest = 0.0;
+    for (int k = 0; k < 3; ++k) widest = fmax(widest, unord(scene[7 + 2 * k]) - unord(scene[6 + 2 * k]));
     for (int k = 0; k < 3; ++k)
     {
-        double lo = unord(scene[k]), hi = unord(scene[3 + k]);
+        double lo, hi;
+        trim_range(unord(scene[k]), unord(scene[3 + k]), unord(scene[6 + 2 * k]), unord(scene[7 + 2 * k]), widest, lo, hi);
         double v = (b.fat[6 * static_cast<size_t>(i) + k] + b.fat[6 * static_cast<size_t>(i) + k + 3]) * 0.5;
         double u = hi > lo ? (v - lo) / (hi - lo) : 0.0;
         u = fmin(fmax(u, 0.0), 1.0);

@@ -169,7 +169,7 @@ struct lbvh_dev
     uint32_t n_chunks, span_levels;
     float4 *span_box;
     float4 *span_tab;
-    unsigned long long *scene; // 6 ordered-integer bounds of leaf centroids
+    unsigned long long *scene; // ordered-integer bounds of leaf centroids (3 lower, 3 upper), then each axis' bulk
     // batched independent worlds (n_worlds > 1): bodies [wstart[w], wstart[w+1]) form
     // world w; Morton keys carry the world in their top wbits bits, so world w's leaves
     // are sorted positions [wstart[w], wstart[w+1]) and the walk prunes other worlds
