@@ -855,9 +855,13 @@ void pkg_ctx::step_once(double dt, hipEvent_t *ev, bool defer_pos)
     // entry, when few pairs are expected (as the last step's; launch_gjk tells why);
     // launch shapes that were set or tuned keep the separate stages.
     const uint64_t expect = last.steps_total ? last.gjk_fp64 + last.gjk_fp64 / 4 : Pn;
-    const bool fused = !trials && !tuned && expect <= kWavePairs;
-    const uint32_t want_hits = fused ? static_cast<uint32_t>(expect) : last_hits + last_hits / 2;
-    size_hits(std::min<uint32_t>(Pn, want_hits));
+    bool fused = !trials && !tuned && expect <= kWavePairs;
+    const uint32_t hits_guess = last_hits + last_hits / 2;
+    size_hits(std::min<uint32_t>(Pn, fused ? static_cast<uint32_t>(expect) : hits_guess));
+    // the fused kernel's wavefronts: at least 2,048 where there are pairs for them (2 a SIMD;
+    // the ones past the list leave at once), so a list longer than expected is not walked by a few
+    const uint32_t waves = std::max<uint32_t>(static_cast<uint32_t>(std::min<uint64_t>(expect, kWavePairs)),
+                                              std::min<uint32_t>(Pn, 2048));
     if (Pn)
     {
         gjk_list.reserve(Pn);
@@ -883,27 +887,29 @@ void pkg_ctx::step_once(double dt, hipEvent_t *ev, bool defer_pos)
         {
             if (again)
                 for (int c : {C_GJK_LIST, C_GJK_LIST2, C_HITS, C_MLIVE, C_EPA_OVF}) reset_counter(c);
-            const gjk_wave_in wv{fused, static_cast<uint32_t>(expect), ovf_list.p};
+            const gjk_wave_in wv{fused, waves, ovf_list.p};
             launch_gjk(keys[nxt].p, Pn, b, s, has_uv, group, g, gjk_list.p, cull_rec.p, f32, wv, mo, counters.p, st);
         };
-        gjk_stage(tune.gjk_group, false);
-        record(ev, 4, st);
-        read_counters(C_HITS, C_MLIVE);
-        uint32_t hits = static_cast<uint32_t>(h_counters[C_HITS]);
-        if (h_counters[C_MLIVE] > live_cap)
-            throw pk_error(PKG_DEVICE_ERROR, "more culled pairs with contacts than manifolds with contacts");
-        // the entries the hit lists need: the hits, or with the fused kernel the listed pairs
-        auto entries = [&]
-        { return static_cast<uint32_t>(h_counters[!fused ? C_HITS : (f32.s32 ? C_GJK_LIST2 : C_GJK_LIST)]); };
-        if (const uint32_t need = entries(); need > g.cap)
+        uint32_t hits = 0;
+        for (int attempt = 0;; ++attempt)
         {
-            // more than the hit lists hold: grow them and run the stage again
-            size_hits(need + need / 4);
-            gjk_stage(tune.gjk_group, true);
+            gjk_stage(tune.gjk_group, attempt > 0);
             record(ev, 4, st);
             read_counters(C_HITS, C_MLIVE);
             hits = static_cast<uint32_t>(h_counters[C_HITS]);
-            if (entries() > g.cap) throw pk_error(PKG_DEVICE_ERROR, "GJK hit count changed between identical runs");
+            if (h_counters[C_MLIVE] > live_cap)
+                throw pk_error(PKG_DEVICE_ERROR, "more culled pairs with contacts than manifolds with contacts");
+            // the entries the hit lists need: the hits, or with the fused kernel the listed
+            // pairs, of which it takes none when they are too many for the lists or for it
+            const uint32_t need =
+                static_cast<uint32_t>(h_counters[!fused ? C_HITS : (f32.s32 ? C_GJK_LIST2 : C_GJK_LIST)]);
+            const bool too_long = fused && need > kWavePairs;
+            if (!too_long && need <= g.cap) break;
+            if (attempt > 2) throw pk_error(PKG_DEVICE_ERROR, "GJK hit count changed between identical runs");
+            // the stage runs again with larger lists, or on a longer list than a wavefront per
+            // pair suits (few pairs before, many now) as separate kernels
+            if (too_long) fused = false;
+            size_hits(too_long ? std::min<uint32_t>(Pn, hits_guess) : need + need / 4);
         }
         last_hits = hits;
         // overflowed solves rerun in larger stores (capacity never changes a result)

@@ -753,7 +753,7 @@ void launch_gjk(const uint64_t *keys, uint32_t n_pairs, const bodies_dev &b, con
     }
     if (wv.on)
     {
-        launch_gjk_epa_wave(keys, list, slot, wv.expect, b, s, uv, g, wv.ovf_list, counters, st);
+        launch_gjk_epa_wave(keys, list, slot, wv.waves, b, s, uv, g, wv.ovf_list, counters, st);
         return;
     }
     // sized for every pair up to kListGrid workgroups, which then step through the list

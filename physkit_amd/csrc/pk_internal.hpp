@@ -273,8 +273,8 @@ struct gjk32_in
     uint32_t *list2;
 };
 // GJK and EPA of every listed pair by a wavefront each (k_wave.hip): entry i of the list is
-// entry i of the hit arrays, and the stage ends with each hit's contact. expect: the pairs
-// expected (sizes the grid; the kernel reads the count).
+// entry i of the hit arrays, and the stage ends with each hit's contact. waves: wavefronts
+// launched, which share the list if it is longer (the kernel reads its count).
 // Longer lists take the separate stages: k_gjk's 32-64 pairs per wavefront then fill the
 // chip and spend less on each (GJK and EPA in ms, separate / fused: 535 sphere, box and hull
 // pairs of 1,934 listed 0.34 / 0.13; 752 of 755 box pairs 0.11 / 0.07; 2,092 of 2,301
@@ -284,10 +284,10 @@ constexpr uint32_t kWavePairs = 8192;
 struct gjk_wave_in
 {
     bool on;
-    uint32_t expect;
+    uint32_t waves;
     uint32_t *ovf_list;
 };
-void launch_gjk_epa_wave(const uint64_t *keys, const uint32_t *list, int list_slot, uint32_t expect, const bodies_dev &b,
+void launch_gjk_epa_wave(const uint64_t *keys, const uint32_t *list, int list_slot, uint32_t waves, const bodies_dev &b,
                          const shapes_dev &s, bool uv, const gjk_out_dev &g, uint32_t *ovf_list,
                          unsigned long long *counters, hipStream_t st);
 // What the cull also settles of the manifold update: a pair whose bodies are apart has

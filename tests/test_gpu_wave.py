@@ -101,3 +101,34 @@ def test_fused_and_separate_stages_agree(pk, kind, n, steps, flags):
     for g in worlds:
         g.close()
     assert hits > 0 or n == 2  # two boxes may not have met yet
+
+
+def test_list_that_grows_at_once(pk):
+    """A step that lists many pairs after one that listed hardly any (bodies set back to a dense
+    state): the same contacts as with separate kernels set, in at most twice their time."""
+    s = pk.scene(pk.SCENE_HULLS, 4713, 65536)
+    ids = np.arange(65536, dtype=np.uint32)
+    rest = {"vel": np.zeros((65536, 3)), "angvel": np.zeros((65536, 3)), "quat": s["quat"]}
+    ms, out = [], []
+    for tuned in (False, True):
+        g = pk.GpuWorld(iterations=4, flags=pk.FLAG_EPA_GUARD)
+        g.load_scene(s)
+        if tuned:
+            g.set_tuning(4, 64, 1 << 20)
+        took = []
+        for _ in range(4):
+            g.set_state(ids, pos=30.0 * s["pos"], **rest)
+            g.step(s["dt"], 2)
+            assert g.counters()["gjk_listed"] < 1000
+            g.set_state(ids, pos=s["pos"], **rest)
+            t = g.step_timed(s["dt"], 1)
+            took.append(t["gjk"] + t["epa"])
+        c = g.counters()
+        assert c["gjk_listed"] > 50000
+        out.append((g.pairs(), *g.manifolds(), g.bodies()["pos"], c["gjk_hits"]))
+        ms.append(min(took))
+        g.close()
+    for i, (a, b) in enumerate(zip(*out)):
+        _assert_same("dense", i, a, b)
+    print(f"[wave] dense step: default {ms[0]:.3f} ms, separate kernels {ms[1]:.3f} ms", flush=True)
+    assert ms[0] <= 2.0 * ms[1]
