@@ -316,13 +316,21 @@ typedef struct pkg_tuning
     float epa_lds_ms[3];   /* EPA stage ms per step with epa_lds_max 0, 4096, 2^32 - 1 */
 } pkg_tuning;
 
+/* By default, where at most 8,192 pairs are expected to need GJK (the last step's number and a
+ * quarter), one kernel runs GJK and EPA, a wavefront per pair, and the GJK and EPA shapes
+ * above are not used. pkg_set_tuning with a gjk_lanes, epa_block or epa_lds_max other than the
+ * current one (unless all three are the defaults) keeps them in separate kernels of those
+ * shapes, and so does pkg_autotune where it finds that faster. */
+
 /* Picks the launch shapes above by timing them on this world. It takes `steps` real
  * steps (the world advances as under pkg_step, with the same results); in each, after
  * the GJK and EPA stages have run, it runs them again with every candidate shape on
  * that step's own pairs and hits (both stages are idempotent) and times each run. It
  * keeps the fastest of each: GJK lanes on the GJK stage, the EPA block size with every
- * batch per thread, then the LDS threshold with the step's fastest block size.
- * pkg_upload_bodies returns to the defaults. out (optional) receives the choice and the
+ * batch per thread, then epa_lds_max with the step's fastest block size; and, over the steps
+ * with at most 8,192 pairs for GJK, whichever is faster of the one kernel and the
+ * fastest separate ones. pkg_upload_bodies returns gjk_lanes and this last choice to the
+ * defaults. out (optional) receives the choice and the
  * mean times measured. */
 pkg_status pkg_autotune(pkg_ctx *ctx, double dt, int steps, pkg_tuning *out);
 pkg_status pkg_get_tuning(pkg_ctx *ctx, pkg_tuning *out);

@@ -293,6 +293,9 @@ struct pkg_ctx
     {
         hipEvent_t t0 = nullptr, t1 = nullptr;
         double gjk[4] = {0, 0, 0, 0}, epa_block[3] = {0, 0, 0}, epa_lds[3] = {0, 0, 0};
+        // steps with lists short enough for it: the fused kernel, and the fastest GJK and
+        // EPA shapes as separate kernels
+        double fused = 0, separate = 0;
     } *trials = nullptr;
     dbuf<double> simplex, info;
     dbuf<uint8_t> status;
@@ -355,7 +358,7 @@ struct pkg_ctx
     // until pkg_upload_bodies loads bodies again
     bool poisoned = false;
     std::vector<uint32_t> h_shape; // shape of each uploaded body (checks shape re-uploads)
-    void update_gjk_group()
+    int default_gjk_group() const
     {
         double cost = 0.0;
         uint32_t live = 0;
@@ -365,7 +368,11 @@ struct pkg_ctx
                 cost += shape_cost[h_shape[i]];
                 ++live;
             }
-        if (!tuned) tune.gjk_group = (live && cost <= 14.0 * live) ? 2 : 4;
+        return (live && cost <= 14.0 * live) ? 2 : 4;
+    }
+    void update_gjk_group()
+    {
+        if (!tuned) tune.gjk_group = default_gjk_group();
     }
 
     lbvh_dev tree();
@@ -853,9 +860,9 @@ void pkg_ctx::step_once(double dt, hipEvent_t *ev, bool defer_pos)
     };
     // One wavefront per pair runs GJK and EPA in one kernel, each list entry its own hit
     // entry, when few pairs are expected (as the last step's; launch_gjk tells why);
-    // launch shapes that were set or tuned keep the separate stages.
+    // GJK or EPA shapes that were set, or found faster by pkg_autotune, keep the separate stages.
     const uint64_t expect = last.steps_total ? last.gjk_fp64 + last.gjk_fp64 / 4 : Pn;
-    bool fused = !trials && !tuned && expect <= kWavePairs;
+    bool fused = !trials && tune.fuse && expect <= kWavePairs;
     const uint32_t hits_guess = last_hits + last_hits / 2;
     size_hits(std::min<uint32_t>(Pn, fused ? static_cast<uint32_t>(expect) : hits_guess));
     // the fused kernel's wavefronts: at least 2,048 where there are pairs for them (2 a SIMD;
@@ -952,7 +959,26 @@ void pkg_ctx::step_once(double dt, hipEvent_t *ev, bool defer_pos)
             };
             static const int lanes[4] = {1, 2, 4, 8}, blocks[3] = {64, 128, 256};
             static const uint32_t lds_max[3] = {0u, 4096u, 0xFFFFFFFFu};
-            for (int c = 0; c < 4; ++c) trials->gjk[c] += timed([&] { gjk_stage(lanes[c], true); });
+            const uint32_t listed = static_cast<uint32_t>(h_counters[f32.s32 ? C_GJK_LIST2 : C_GJK_LIST]);
+            const bool is_short = listed <= kWavePairs;
+            double fused_ms = 0, gjk_ms[4];
+            if (is_short) // first: the stages timed after it leave the hit lists as they were
+            {
+                for (int c : {C_EPA_OVF2, C_EPA_BIG_FAIL}) reset_counter(c);
+                size_hits(std::max(listed, hits));
+                fused = true;
+                fused_ms = timed([&] { gjk_stage(tune.gjk_group, true); });
+                fused = false;
+                read_counters(C_HITS, C_MLIVE);
+                if (h_counters[C_HITS] != hits) throw pk_error(PKG_DEVICE_ERROR, "GJK hit count changed between runs");
+                if (const uint32_t novf = static_cast<uint32_t>(h_counters[C_EPA_OVF]))
+                    fused_ms += timed([&] { epa_reruns(novf); });
+            }
+            for (int c = 0; c < 4; ++c)
+            {
+                gjk_ms[c] = timed([&] { gjk_stage(lanes[c], true); });
+                trials->gjk[c] += gjk_ms[c];
+            }
             if (read_counter(C_HITS) != hits) throw pk_error(PKG_DEVICE_ERROR, "GJK hit count changed between runs");
             tuning tu = tune;
             tu.epa_lds_max = 0; // every batch through k_epa while its block size is timed
@@ -969,7 +995,13 @@ void pkg_ctx::step_once(double dt, hipEvent_t *ev, bool defer_pos)
             for (int c = 0; c < 3; ++c)
             {
                 tu.epa_lds_max = lds_max[c];
-                trials->epa_lds[c] += timed([&] { epa_stage(tu, true); });
+                ms[c] = timed([&] { epa_stage(tu, true); });
+                trials->epa_lds[c] += ms[c];
+            }
+            if (is_short)
+            {
+                trials->fused += fused_ms;
+                trials->separate += *std::min_element(gjk_ms, gjk_ms + 4) + *std::min_element(ms, ms + 3);
             }
         }
         // a manifold is non-empty only if its pair had contacts or has a hit now: the
@@ -1429,7 +1461,9 @@ pkg_status pkg_upload_bodies(pkg_ctx *ctx, uint32_t n, const pkg_body_desc *d)
     PKG_GUARD(ctx, {
         ctx->h_static.assign(d->is_static, d->is_static + n);
         ctx->h_shape.assign(d->shape, d->shape + n);
-        ctx->tuned = false; // a new body set: back to the default shapes until tuned again
+        // a new body set: GJK lanes and the fused kernel as by default until tuned again
+        ctx->tuned = false;
+        ctx->tune.fuse = true;
         ctx->update_gjk_group();
         ctx->jcoloured = false;
         hipStream_t st = ctx->st;
@@ -1985,6 +2019,10 @@ pkg_status pkg_set_tuning(pkg_ctx *ctx, const pkg_tuning *t)
         ctx->err = "pkg_set_tuning: tree_refits must be at most 64";
         return PKG_INVALID_ARG;
     }
+    // other GJK or EPA shapes than before: one kernel for both only if they are the defaults
+    const tuning d{};
+    if (g != ctx->tune.gjk_group || e != ctx->tune.epa_block || t->epa_lds_max != ctx->tune.epa_lds_max)
+        ctx->tune.fuse = g == ctx->default_gjk_group() && e == d.epa_block && t->epa_lds_max == d.epa_lds_max;
     ctx->tune.gjk_group = g;
     ctx->tune.epa_block = e;
     ctx->tune.epa_lds_max = t->epa_lds_max;
@@ -2031,6 +2069,7 @@ pkg_status pkg_autotune(pkg_ctx *ctx, double dt, int steps, pkg_tuning *out)
             tu.gjk_group = lanes[argmin(tr.gjk, 4)];
             tu.epa_block = blocks[argmin(tr.epa_block, 3)];
             tu.epa_lds_max = lds_max[argmin(tr.epa_lds, 3)];
+            tu.fuse = tr.fused <= tr.separate; // no short list seen: as by default
             for (int c = 0; c < 4; ++c) res.gjk_ms[c] = static_cast<float>(tr.gjk[c] / steps);
             for (int c = 0; c < 3; ++c)
             {

@@ -276,10 +276,13 @@ struct gjk32_in
 // entry i of the hit arrays, and the stage ends with each hit's contact. waves: wavefronts
 // launched, which share the list if it is longer (the kernel reads its count).
 // Longer lists take the separate stages: k_gjk's 32-64 pairs per wavefront then fill the
-// chip and spend less on each (GJK and EPA in ms, separate / fused: 535 sphere, box and hull
-// pairs of 1,934 listed 0.34 / 0.13; 752 of 755 box pairs 0.11 / 0.07; 2,092 of 2,301
-// 0.70 / 0.48; 17,879 of 17,886 box pairs 0.23 / 0.29; 56,165 of 84,521 1.09 / 1.17;
-// 143,064 of 361,508 hull pairs 2.9 / 4.3).
+// chip and spend less on each. GJK and EPA in ms, separate / fused, by pairs listed: hulls
+// (4 in 10 hit) 1,433 0.15 / 0.09, 2,739 0.16 / 0.09, 4,128 0.16 / 0.09, 5,530 0.17 / 0.12,
+// 143,064 of 361,508 2.9 / 4.3; sphere, box and hull pairs of batched worlds (6 in 10) 334
+// 0.34 / 0.15, 1,941 0.44 / 0.23, 6,557 0.50 / 0.29, 7,813 0.52 / 0.34, 84,521 1.09 / 1.17;
+// boxes (all hit) 719 0.10 / 0.06, 2,239 0.12 / 0.08, 5,027 0.13 / 0.12, 5,836 0.13 / 0.13,
+// 6,312 0.13 / 0.14, 17,886 0.23 / 0.29. The line is on the pairs expected, the last step's
+// and a quarter: 6,553 listed pairs.
 constexpr uint32_t kWavePairs = 8192;
 struct gjk_wave_in
 {
@@ -316,6 +319,7 @@ struct tuning
     uint32_t epa_lds_max = 0xFFFFFFFFu; // batches of at most this many GJK hits run one EPA solve per
                                         // wavefront (k_epa_wave); larger ones one per thread (k_epa)
     uint32_t tree_refits = 7;    // steps that refit the last LBVH hierarchy between full builds
+    bool fuse = true; // lists expected to be short run GJK and EPA in one kernel (kWavePairs)
 };
 void launch_epa(const uint64_t *keys, uint32_t n_hits, const bodies_dev &b, const shapes_dev &s, bool uv,
                 const tuning &tu, gjk_out_dev &g, uint32_t *ovf_list, unsigned long long *counters, hipStream_t st);

@@ -161,3 +161,39 @@ def test_epa_tiers_and_overflows_bitexact(pk, oracle):
         if lds == 0:
             assert g.counters()["epa_overflow"] > 0, "no solve outgrew the first tier's store"
         g.close()
+
+
+def test_short_lists_keep_the_fused_kernel(pk):
+    """1,024 boxes two seconds in, a few hundred pairs through GJK, where one kernel for GJK and EPA
+    is the faster form (its EPA stage then only waits): it stays in use when only tree_refits
+    is set, when the defaults are set again, and after pkg_autotune; other shapes end it."""
+    s = pk.scene(pk.SCENE_BOXES, 905, 1024)
+
+    def epa_ms(*setup):
+        g = pk.GpuWorld(iterations=s["iterations"], flags=s["flags"] | pk.FLAG_EPA_GUARD)
+        g.load_scene(s)
+        g.step(s["dt"], 120)
+        for f in setup:
+            f(g)
+        assert 0 < g.counters()["gjk_fp64"] < 4096
+        ms = min(g.step_timed(s["dt"], 1)["epa"] for _ in range(8))
+        state = _state(g)
+        g.close()
+        return ms, state
+
+    def shapes(refits=None, lds=None):
+        def f(g):
+            t = g.tuning()
+            g.set_tuning(t["gjk_lanes"], t["epa_block"], t["epa_lds_max"] if lds is None else lds, refits)
+        return f
+
+    separate, want = epa_ms(shapes(lds=1 << 20))
+    for name, setup in (("refits", [shapes(refits=5)]), ("defaults again", [shapes(lds=0), shapes(lds=0xFFFFFFFF)]),
+                        ("default", [])):
+        ms, got = epa_ms(*setup)
+        print(f"[tuning] {name}: EPA stage {ms:.4f} ms, separate kernels {separate:.4f} ms", flush=True)
+        assert ms < 0.5 * separate, name
+        _same(name, got, want)
+    ms, _ = epa_ms(lambda g: g.autotune(s["dt"], 8))
+    print(f"[tuning] autotune: EPA stage {ms:.4f} ms", flush=True)
+    assert ms < 0.5 * separate
