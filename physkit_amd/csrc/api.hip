@@ -344,10 +344,11 @@ struct pkg_ctx
     dbuf<uint32_t> q_out_id, q_world;
     hipEvent_t q_ev[2] = {nullptr, nullptr}; // query kernel timing
 
-    // body state on its way between the caller's arrays and the device: two halves of pinned
-    // memory and of device memory, grown on use up to kXferHalf each, kept until the ctx ends
+    // body state on its way between the caller's arrays and the device: pinned memory and
+    // (above kXferDirect) device memory, doubled on use up to two halves of kXferHalf and kept
+    // until the ctx ends
     char *xfer_pin = nullptr;
-    size_t xfer_half = 0;
+    size_t xfer_cap = 0;
     dbuf<char> xfer_dev;
     hipEvent_t xfer_ev[2] = {nullptr, nullptr};
     void xfer_reserve(size_t bytes);
@@ -505,24 +506,24 @@ void record(hipEvent_t *ev, int k, hipStream_t st)
 }
 } // namespace
 
-// Up to this many bytes of body state the kernels read and write the pinned memory
+// Up to kXferDirect bytes of body state the kernels read and write the pinned memory
 // themselves (one launch and one wait: 64 bodies downloaded in 0.03 ms); more goes through
-// device memory and the copy engine in halves, the host's copy of one half overlapping the
-// transfer of the other.
+// device memory and the copy engine, up to kXferHalf in one piece, above that in halves, the
+// host's copy of one half overlapping the transfer of the other.
 constexpr size_t kXferDirect = 256 << 10, kXferHalf = 16 << 20;
 void pkg_ctx::xfer_reserve(size_t bytes)
 {
     for (auto &e : xfer_ev)
         if (!e) hip_check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "event create");
-    if (bytes > kXferDirect) xfer_dev.reserve(2 * kXferHalf);
-    size_t half = kXferDirect;
-    if (bytes > half) half = kXferHalf;
-    if (half <= xfer_half) return;
+    size_t want = kXferDirect;
+    while (want < bytes && want < 2 * kXferHalf) want *= 2;
+    if (bytes > kXferDirect) xfer_dev.reserve(want);
+    if (want <= xfer_cap) return;
     if (xfer_pin) (void)hipHostFree(xfer_pin);
     xfer_pin = nullptr;
-    xfer_half = 0;
-    hip_check(hipHostMalloc(reinterpret_cast<void **>(&xfer_pin), 2 * half), "pinned alloc");
-    xfer_half = half;
+    xfer_cap = 0;
+    hip_check(hipHostMalloc(reinterpret_cast<void **>(&xfer_pin), want), "pinned alloc");
+    xfer_cap = want;
 }
 
 lbvh_dev pkg_ctx::tree()
@@ -1886,13 +1887,13 @@ pkg_status pkg_set_body_state(pkg_ctx *ctx, uint32_t count, const uint32_t *ids,
         ctx->xfer_reserve(rec * count);
         const bool direct = rec * count <= kXferDirect;
         // records per half, a multiple of 64 so every array of a half starts aligned
-        const uint32_t per = direct ? count : static_cast<uint32_t>(std::min<size_t>(kXferHalf / rec / 64 * 64, count));
+        const uint32_t per = rec * count <= kXferHalf ? count : static_cast<uint32_t>(kXferHalf / rec / 64 * 64);
         for (uint32_t first = 0, round = 0; first < count; first += per, ++round)
         {
             const uint32_t n = std::min(per, count - first), h = round & 1;
             // the half's last transfer has left the pinned memory
             if (round > 1) hip_check(hipEventSynchronize(ctx->xfer_ev[h]), "event sync");
-            char *pin = ctx->xfer_pin + h * ctx->xfer_half;
+            char *pin = ctx->xfer_pin + h * kXferHalf;
             char *dev = direct ? pin : ctx->xfer_dev.p + h * kXferHalf;
             std::vector<host_part> parts;
             const double *d[4] = {};
@@ -2103,7 +2104,7 @@ pkg_status pkg_download_bodies(pkg_ctx *ctx, const pkg_body_state *out)
         if (!n || !rec) return PKG_OK;
         ctx->xfer_reserve(rec * n);
         const bool direct = rec * n <= kXferDirect;
-        const uint32_t per = direct ? n : static_cast<uint32_t>(std::min<size_t>(kXferHalf / rec / 64 * 64, n));
+        const uint32_t per = rec * n <= kXferHalf ? n : static_cast<uint32_t>(kXferHalf / rec / 64 * 64);
         std::vector<host_part> parts[2];
         const uint32_t rounds = (n + per - 1) / per;
         for (uint32_t round = 0; round <= rounds; ++round)
@@ -2111,7 +2112,7 @@ pkg_status pkg_download_bodies(pkg_ctx *ctx, const pkg_body_state *out)
             if (round < rounds)
             {
                 const uint32_t first = round * per, count = std::min(per, n - first), h = round & 1;
-                char *pin = ctx->xfer_pin + h * ctx->xfer_half;
+                char *pin = ctx->xfer_pin + h * kXferHalf;
                 char *dev = direct ? pin : ctx->xfer_dev.p + h * kXferHalf;
                 char *to[6] = {};
                 size_t at = 0;

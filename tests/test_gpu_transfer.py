@@ -57,3 +57,51 @@ def test_download_and_set_state(pk, n):
     for f in ("pos", "vel", "angvel", "quat"):
         np.testing.assert_array_equal(b[f], s[f])
     g.close()
+
+
+def test_transfer_memory_follows_the_call(pk):
+    """What a context keeps for its transfers is at most four times a call's bytes, in pinned and in
+    device memory, not the largest call's: 8 contexts of 1,800 bodies (269 KiB down) hold at
+    most 8 MiB of device memory for them (and one granule of 2 MiB each)."""
+    from test_zz_no_alloc import Hip
+    hip = Hip().L
+
+    def free():
+        assert hip.hipDeviceSynchronize() == 0
+        f, t = C.c_size_t(), C.c_size_t()
+        assert hip.hipMemGetInfo(C.byref(f), C.byref(t)) == 0
+        return f.value
+
+    worlds = []
+    for k in range(8):
+        worlds.append(pk.GpuWorld())
+        worlds[-1].load_scene(_scene(pk, 1800))
+    before = free()
+    got = [g.bodies()["pos"] for g in worlds]
+    used = before - free()
+    print(f"[transfer] {used / 2**20:.1f} MiB of device memory for 8 contexts' transfers", flush=True)
+    assert used <= (8 + 16) << 20
+    want = _scene(pk, 1800)["pos"]
+    for g, p in zip(worlds, got):
+        np.testing.assert_array_equal(p, want)
+        g.close()
+
+
+def test_growing_and_shrinking_calls(pk):
+    """One context whose calls go up and down over every size of the kept memory."""
+    n = 230000
+    s = _scene(pk, n)
+    g = pk.GpuWorld()
+    g.load_scene(s)
+    rng = np.random.default_rng(6)
+    want = s["vel"].copy()
+    for count in (1, 9362, 9363, 3000, 20000, 599186, 180000, 64, 230000):
+        ids = rng.permutation(n)[:min(count, n)].astype(np.uint32)
+        v = rng.normal(size=(len(ids), 3))
+        g.set_state(ids, vel=v)
+        want[ids] = v
+        got = np.full((n, 3), -1.0)
+        st = pk.pkg_body_state(vel=got.ctypes.data_as(pk.D))
+        assert g.L.pkg_download_bodies(g.h, C.byref(st)) == 0
+        np.testing.assert_array_equal(got, want)
+    g.close()
