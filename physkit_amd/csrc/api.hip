@@ -6,6 +6,7 @@
 // pair count, GJK hit count, EPA overflow count, solver rows, colour rounds.
 #include "physkit_amd.h"
 #include "pk_access.hpp"
+#include "pk_copy.hpp"
 #include "pk_gjk.hpp"
 #include "uv_sphere.hpp"
 
@@ -17,8 +18,6 @@
 #include <mutex>
 #include <stdexcept>
 #include <string>
-#include <system_error>
-#include <thread>
 #include <vector>
 
 namespace
@@ -122,44 +121,6 @@ __global__ void k_export(bodies_dev b, uint32_t first, uint32_t count, export_to
     records(o.quat, b.quat, 4);
     if (o.fat && t < 6 * count) o.fat[t] = b.fat[6 * static_cast<size_t>(first) + t];
     if (o.moved && t < count) o.moved[t] = b.moved[first + t];
-}
-
-// host memory parts copied together, split over a few threads when large (a fresh array's
-// pages are faulted in by whoever writes them first)
-struct host_part
-{
-    char *dst;
-    const char *src;
-    size_t bytes;
-};
-void copy_parts(const std::vector<host_part> &parts)
-{
-    size_t total = 0;
-    for (const host_part &p : parts) total += p.bytes;
-    auto range = [&](size_t lo, size_t hi)
-    {
-        size_t at = 0;
-        for (const host_part &p : parts)
-        {
-            const size_t a = std::max(lo, at), e = std::min(hi, at + p.bytes);
-            if (a < e) std::memcpy(p.dst + (a - at), p.src + (a - at), e - a);
-            at += p.bytes;
-        }
-    };
-    const size_t n = std::min<size_t>(std::min<size_t>(8, std::thread::hardware_concurrency()), total >> 20);
-    if (n < 2) return range(0, total);
-    std::vector<std::thread> team;
-    team.reserve(n - 1);
-    size_t done = 0; // the parts given to threads; the rest, also after a thread could not start, is copied here
-    try
-    {
-        for (; done + 1 < n; ++done) team.emplace_back(range, total / n * done, total / n * (done + 1));
-    }
-    catch (const std::system_error &)
-    {
-    }
-    range(total / n * done, total);
-    for (std::thread &t : team) t.join();
 }
 
 int id_bits(uint32_t n)
