@@ -742,6 +742,7 @@ __device__ __forceinline__ int epa_solve(const shape &w, simplex &x, store<K> &s
         }
         if (e.heaped) e.push_range(base, end);
         e.nfaces = end;
+        lds_sync(); // point pi, which every lane may read from here on
     }
     const int mf = e.nearest(it);
     if (mf < 0) return 0;
