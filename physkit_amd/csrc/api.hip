@@ -1049,7 +1049,7 @@ void pkg_ctx::step_once(double dt, hipEvent_t *ev, bool defer_pos)
                 longest = static_cast<uint32_t>(std::min<unsigned long long>(h_counters[C_ISL_MAX], 0xFFFFFFFFull));
                 if (nl && longest <= static_cast<uint32_t>(f32 ? kChunkMax32 : kChunkMax))
                 {
-                    const uint32_t *ord = clist.p, *isl = nullptr;
+                    const uint32_t *ord = clist.p, *isl = nullptr, *root = iroot.p;
                     if (nl > static_cast<uint32_t>(kChunkTwoLanes))
                     {
                         ibase.reserve(std::max<uint32_t>(n, 1));
@@ -1058,10 +1058,10 @@ void pkg_ctx::step_once(double dt, hipEvent_t *ev, bool defer_pos)
                         launch_island_group(clist.p, nl, icnt.p, n, iroot.p, irank.p, ibase.p, iv.p, iv_alt.p, counters.p,
                                             st);
                         ord = iv.p;
-                        isl = iv_alt.p;
+                        isl = root = iv_alt.p;
                     }
                     record(ev, 10, st);
-                    launch_solve_chunks(keys[nxt].p, ord, isl, nl, longest, b, MF(nxt), colour.p, wo, pb,
+                    launch_solve_chunks(keys[nxt].p, ord, isl, root, nl, longest, b, MF(nxt), colour.p, wo, pb,
                                         cfg.solver_iterations, dt, thr, f32, counters.p, st);
                     record(ev, 11, st);
                     solved = chunked = true;

@@ -163,6 +163,13 @@ template <class T, class V, int S> struct row_t
     V n, r[S]; // r is kept in LDS between colours where a lane holds both sides
     T a, meff, bias, i11, i12, i22, an, a1, a2;
 };
+// The FP32 solve of an island of more than kIslandMaxColours colours: the tangents and Jacobians
+// themselves, computed in FP64 and rounded once, as the per-colour launches keep them
+template <int S> struct row32_t
+{
+    f3 n, t1, t2, jn[S], j1[S], j2[S];
+    float meff, bias, i11, i12, i22, an, a1, a2;
+};
 
 // row_apply and friction_block (pk_solver.hpp) with the Jacobians rebuilt by the operations
 // of basis and make_row
@@ -249,22 +256,12 @@ __device__ __forceinline__ void solve_rows(row_t<double, v3, S> &k, double mu, b
             b[s].ang = b[s].ang + mul(b[s].I, j1[s] * d1 + j2[s] * d2);
         }
 }
-// the FP32 solve: row arithmetic in FP32, increments added to the FP64 velocities
-template <int S>
-__device__ __forceinline__ void solve_rows(row_t<float, f3, S> &k, float mu, bool warm, side32 (&b)[S])
+// the FP32 solve: row arithmetic in FP32, increments added to the FP64 velocities. k: impulses, mass,
+// bias and friction block of the rows along n, t1 and t2
+template <int S, class K>
+__device__ __forceinline__ void apply_rows32(K &k, f3 n, f3 t1, f3 t2, const f3 (&jn)[S], const f3 (&j1)[S],
+                                             const f3 (&j2)[S], float mu, bool warm, side32 (&b)[S])
 {
-    const float sign = copysignf(1.0f, k.n.z);
-    const float bb = k.n.x * k.n.y * k.a;
-    const f3 t1 = f3m(1.0f + sign * k.n.x * k.n.x * k.a, sign * bb, -sign * k.n.x);
-    const f3 t2 = f3m(bb, sign + k.n.y * k.n.y * k.a, -k.n.y);
-    f3 jn[S], j1[S], j2[S];
-#pragma unroll
-    for (int s = 0; s < S; ++s)
-    {
-        jn[s] = flip<S>(fcr(k.r[s], k.n), s);
-        j1[s] = flip<S>(fcr(k.r[s], t1), s);
-        j2[s] = flip<S>(fcr(k.r[s], t2), s);
-    }
     auto push = [&](int s, f3 lin, f3 ang)
     {
         if (b[s].stat) return;
@@ -276,7 +273,7 @@ __device__ __forceinline__ void solve_rows(row_t<float, f3, S> &k, float mu, boo
 #pragma unroll
         for (int s = 0; s < S; ++s)
         {
-            if (k.an != 0.0f) push(s, scl(k.n, k.an), scl(jn[s], k.an));
+            if (k.an != 0.0f) push(s, scl(n, k.an), scl(jn[s], k.an));
             if (k.a1 != 0.0f) push(s, scl(t1, k.a1), scl(j1[s], k.a1));
             if (k.a2 != 0.0f) push(s, scl(t2, k.a2), scl(j2[s], k.a2));
         }
@@ -286,7 +283,7 @@ __device__ __forceinline__ void solve_rows(row_t<float, f3, S> &k, float mu, boo
 #pragma unroll
     for (int s = 0; s < S; ++s)
     {
-        x[s] = dotf(k.n, to_f3(b[s].vel));
+        x[s] = dotf(n, to_f3(b[s].vel));
         y[s] = dotf(jn[s], to_f3(b[s].ang));
     }
     const float jv = jv_sum(x, y);
@@ -299,7 +296,7 @@ __device__ __forceinline__ void solve_rows(row_t<float, f3, S> &k, float mu, boo
 #pragma unroll
     for (int s = 0; s < S; ++s)
     {
-        push(s, scl(k.n, ap), scl(jn[s], ap));
+        push(s, scl(n, ap), scl(jn[s], ap));
         const f3 vel = to_f3(b[s].vel), ang = to_f3(b[s].ang);
         x[s] = dotf(t1, vel);
         y[s] = dotf(j1[s], ang);
@@ -321,6 +318,27 @@ __device__ __forceinline__ void solve_rows(row_t<float, f3, S> &k, float mu, boo
 #pragma unroll
     for (int s = 0; s < S; ++s) push(s, addf(scl(t1, d1), scl(t2, d2)), addf(scl(j1[s], d1), scl(j2[s], d2)));
 }
+// the Jacobians rebuilt in FP32 from the rounded normal and arms
+template <int S>
+__device__ __forceinline__ void solve_rows(row_t<float, f3, S> &k, float mu, bool warm, side32 (&b)[S])
+{
+    const float sign = copysignf(1.0f, k.n.z);
+    const float bb = k.n.x * k.n.y * k.a;
+    const f3 t1 = f3m(1.0f + sign * k.n.x * k.n.x * k.a, sign * bb, -sign * k.n.x);
+    const f3 t2 = f3m(bb, sign + k.n.y * k.n.y * k.a, -k.n.y);
+    f3 jn[S], j1[S], j2[S];
+#pragma unroll
+    for (int s = 0; s < S; ++s)
+    {
+        jn[s] = flip<S>(fcr(k.r[s], k.n), s);
+        j1[s] = flip<S>(fcr(k.r[s], t1), s);
+        j2[s] = flip<S>(fcr(k.r[s], t2), s);
+    }
+    apply_rows32<S>(k, k.n, t1, t2, jn, j1, j2, mu, warm, b);
+}
+template <int S>
+__device__ __forceinline__ void solve_rows(row32_t<S> &k, float mu, bool warm, side32 (&b)[S])
+{ apply_rows32<S>(k, k.n, k.t1, k.t2, k.jn, k.j1, k.j2, mu, warm, b); }
 
 __device__ __forceinline__ void put_side(side64 &d, double im, const m3 &I)
 {
@@ -354,23 +372,29 @@ __device__ __forceinline__ uint16_t slot_of(const uint32_t *ids, uint32_t n_ids,
 // Chunk k: the islands whose first position lies in [k window, (k + 1) window) of the island
 // order (isl null: the whole list is one chunk). With islands of at most `longest`
 // manifolds a chunk has at most window + longest - 1, which the launch keeps within CAP and
-// within the workgroup's lanes (LANES per manifold).
-template <bool F32, int LANES, int CAP>
+// within the workgroup's lanes (LANES per manifold). root: the island root at each position.
+// In the FP32 solve, islands of more than kIslandMaxColours colours are left to a second launch
+// (DEEP), which takes only those and keeps their rows as row32_t (208 registers; the others need
+// 171); C_DEEP counts the chunks that have any.
+template <bool F32, int LANES, int CAP, bool DEEP>
 __global__ void __launch_bounds__(LANES *CAP)
-    k_solve_chunks(const uint64_t *keys, const uint32_t *ord, const uint32_t *isl, uint32_t nl, uint32_t window,
-                   bodies_dev b, manifolds_dev m, uint32_t *colour, const uint32_t *world_of, const uint32_t *pair_base,
-                   uint32_t iters, double dt, double thr, unsigned long long *counters)
+    k_solve_chunks(const uint64_t *keys, const uint32_t *ord, const uint32_t *isl, const uint32_t *root, uint32_t nl,
+                   uint32_t window, bodies_dev b, manifolds_dev m, uint32_t *colour, const uint32_t *world_of,
+                   const uint32_t *pair_base, uint32_t iters, double dt, double thr, unsigned long long *counters)
 {
     constexpr int S = 3 - LANES;
     using T = typename std::conditional<F32, float, double>::type;
     using V = typename std::conditional<F32, f3, v3>::type;
     using side = typename std::conditional<F32, side32, side64>::type;
+    static_assert(!DEEP || (F32 && LANES == 2));
+    if (DEEP && counters[C_DEEP] == 0) return;
     __shared__ uint32_t ids[2 * CAP];
     __shared__ double lv[2 * CAP][6]; // velocities; before them, the colouring's claims and taken colours
     // both sides' lever arms where one lane has them: with them the rows of four contacts
     // would not fit its registers
     __shared__ double arms[LANES == 1 ? 24 : 1][LANES == 1 ? CAP : 1];
     __shared__ uint32_t lim[3];
+    __shared__ uint32_t deep[F32 ? 2 * CAP / 32 : 1]; // a bit per body slot: the root of an island left to DEEP
     const uint32_t tid = threadIdx.x, threads = blockDim.x;
     uint32_t s0 = 0, e0 = nl;
     if (tid < 3) lim[tid] = tid < 2 ? nl : 0u;
@@ -426,7 +450,7 @@ __global__ void __launch_bounds__(LANES *CAP)
         }
     // this lane's manifold and sides
     uint32_t i = tid / LANES;
-    const bool own = i < cnt;
+    bool own = i < cnt;
     uint32_t p = 0, id[2] = {0, 0}, mine[S];
     side body[S];
     uint16_t slot[S];
@@ -506,8 +530,20 @@ __global__ void __launch_bounds__(LANES *CAP)
         if (tid % LANES == 0) colour[p] = col;
     }
     __syncthreads();
-    const uint32_t n_colours = lim[2];
+    uint32_t n_colours = lim[2];
+    const bool any_deep = F32 && n_colours > kIslandMaxColours;
+    if (DEEP && !any_deep) return;
     if (tid == 0) atomicMax(&counters[C_NCOL], static_cast<unsigned long long>(n_colours));
+    auto root_bit = [&]
+    { return slot_of(ids, n_ids, root[s0 + i]); };
+    if (any_deep)
+    {
+        if (tid < 2 * CAP / 32) deep[tid] = 0;
+        __syncthreads();
+        if (own && col >= kIslandMaxColours) atomicOr(&deep[root_bit() >> 5], 1u << (root_bit() & 31u));
+        if (!DEEP && tid == 0) atomicAdd(&counters[C_DEEP], 1ull);
+        __syncthreads();
+    }
     if (threads > 64)
     {
         // Manifolds handed out again by colour, so that a colour's are in few wavefronts:
@@ -541,6 +577,11 @@ __global__ void __launch_bounds__(LANES *CAP)
         }
         __syncthreads();
     }
+    if (any_deep)
+    {
+        if (own) own = ((deep[root_bit() >> 5] >> (root_bit() & 31u)) & 1u) == (DEEP ? 1u : 0u);
+        if (!DEEP) n_colours = kIslandMaxColours;
+    }
     // velocities
     for (uint32_t t = tid; t < n_ids; t += threads)
     {
@@ -557,7 +598,7 @@ __global__ void __launch_bounds__(LANES *CAP)
         }
     }
     // rows: build_contact_jacobian (:874-953) and setup_contacts (:1075-1102)
-    row_t<T, V, S> k[4];
+    typename std::conditional<DEEP, row32_t<S>, row_t<T, V, S>>::type k[4];
     uint32_t valid = 0, sl = 0;
     T mu = 0;
     if (own)
@@ -639,10 +680,21 @@ __global__ void __launch_bounds__(LANES *CAP)
                 i12 = 0.0;
             }
             put_v(k[c].n, n);
+            if constexpr (DEEP)
+            {
+                put_v(k[c].t1, t1);
+                put_v(k[c].t2, t2);
+            }
 #pragma unroll
             for (int s = 0; s < S; ++s)
             {
-                if constexpr (LANES == 1)
+                if constexpr (DEEP)
+                {
+                    put_v(k[c].jn[s], flip<S>(cross(r[s], n), s));
+                    put_v(k[c].j1[s], flip<S>(cross(r[s], t1), s));
+                    put_v(k[c].j2[s], flip<S>(cross(r[s], t2), s));
+                }
+                else if constexpr (LANES == 1)
                 {
                     arms[6 * c + 3 * s][tid] = r[s].x;
                     arms[6 * c + 3 * s + 1][tid] = r[s].y;
@@ -651,7 +703,7 @@ __global__ void __launch_bounds__(LANES *CAP)
                 else
                     put_v(k[c].r[s], r[s]);
             }
-            k[c].a = basis_factor(k[c].n);
+            if constexpr (!DEEP) k[c].a = basis_factor(k[c].n);
             k[c].meff = static_cast<T>(meff);
             k[c].bias = static_cast<T>(smin(baum, rbias));
             k[c].i11 = static_cast<T>(i11);
@@ -749,10 +801,10 @@ void launch_island_group(const uint32_t *list, uint32_t nl, const uint32_t *cnt,
     k_island_scatter<<<grid(nl), kBlock, 0, st>>>(list, nl, root_of, rank_of, base, ord, isl);
 }
 
-void launch_solve_chunks(const uint64_t *keys, const uint32_t *ord, const uint32_t *isl, uint32_t nl, uint32_t longest,
-                         const bodies_dev &b, const manifolds_dev &m, uint32_t *colour, const uint32_t *world_of,
-                         const uint32_t *pair_base, uint32_t iters, double dt, double thr, bool f32,
-                         unsigned long long *counters, hipStream_t st)
+void launch_solve_chunks(const uint64_t *keys, const uint32_t *ord, const uint32_t *isl, const uint32_t *root, uint32_t nl,
+                         uint32_t longest, const bodies_dev &b, const manifolds_dev &m, uint32_t *colour,
+                         const uint32_t *world_of, const uint32_t *pair_base, uint32_t iters, double dt, double thr,
+                         bool f32, unsigned long long *counters, hipStream_t st)
 {
     if (!nl) return;
     auto go = [&](auto f, auto lanes, auto capacity)
@@ -767,8 +819,12 @@ void launch_solve_chunks(const uint64_t *keys, const uint32_t *ord, const uint32
         }
         const unsigned threads = (std::min<uint32_t>(most, CAP) * L + 63) / 64 * 64;
         const unsigned nb = isl ? ((nl + window - 1) / window + 7) / 8 * 8 : 1u;
-        k_solve_chunks<F, L, CAP><<<nb, threads, 0, st>>>(keys, ord, isl, nl, window, b, m, colour, world_of, pair_base, iters,
-                                                          dt, thr, counters);
+        k_solve_chunks<F, L, CAP, false><<<nb, threads, 0, st>>>(keys, ord, isl, root, nl, window, b, m, colour, world_of,
+                                                                 pair_base, iters, dt, thr, counters);
+        if constexpr (F)
+            if (longest > kIslandMaxColours) // a colour takes a manifold of the island's
+                k_solve_chunks<F, L, CAP, true><<<nb, threads, 0, st>>>(keys, ord, isl, root, nl, window, b, m, colour,
+                                                                        world_of, pair_base, iters, dt, thr, counters);
     };
     using std::integral_constant;
     using std::bool_constant;

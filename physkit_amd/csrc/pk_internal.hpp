@@ -99,6 +99,7 @@ enum counter_slot
     C_MLIVE = 20,     // pairs listed for the manifold update (see launch_manifold_update)
     C_MLEAF = 21,     // leaves listed for the pair query (dynamic and moved)
     C_EPA_OVF2 = 22,  // overflows of the 512-face store, rerun in global memory
+    C_DEEP = 23,      // FP32 island chunks of more than kIslandMaxColours colours
     // pair query cursors: one per output region, each in its own 256-byte line, so
     // wavefronts reserving output space spread their atomics over kPairRegions
     // addresses instead of serialising on one
@@ -430,16 +431,17 @@ void launch_island_group(const uint32_t *list, uint32_t nl, const uint32_t *cnt,
                          const uint32_t *rank_of, uint32_t *base, uint32_t *ord, uint32_t *isl,
                          unsigned long long *counters, hipStream_t st);
 // The whole contact solve of islands of at most kChunkMax manifolds (kChunkMax32 for the FP32
-// solve, whose longer islands keep the row arithmetic of launch_solve_islands). isl null: the
-// list (at most kChunkTwoLanes) is one chunk. Two lanes per manifold up to 256 manifolds: 512
+// solve, whose longer islands keep the row arithmetic of launch_solve_islands, and whose islands of
+// more than kIslandMaxColours colours that of launch_solve_colour32). isl null: the list (at most
+// kChunkTwoLanes) is one chunk. root: each position's island root. Two lanes per manifold up to 256 manifolds: 512
 // threads, the most whose FP64 rows of four contacts fit the 256 registers a thread then has;
 // one lane, with its lever arms in LDS, up to 512.
 constexpr int kChunkTwoLanes = 256, kChunkMax = 512, kChunkMax32 = 256;
 constexpr uint32_t kChunkFill = 32; // manifolds a chunk takes before another workgroup is opened
-void launch_solve_chunks(const uint64_t *keys, const uint32_t *ord, const uint32_t *isl, uint32_t nl, uint32_t longest,
-                         const bodies_dev &b, const manifolds_dev &m, uint32_t *colour, const uint32_t *world_of,
-                         const uint32_t *pair_base, uint32_t iters, double dt, double thr, bool f32,
-                         unsigned long long *counters, hipStream_t st);
+void launch_solve_chunks(const uint64_t *keys, const uint32_t *ord, const uint32_t *isl, const uint32_t *root, uint32_t nl,
+                         uint32_t longest, const bodies_dev &b, const manifolds_dev &m, uint32_t *colour,
+                         const uint32_t *world_of, const uint32_t *pair_base, uint32_t iters, double dt, double thr,
+                         bool f32, unsigned long long *counters, hipStream_t st);
 // Longer islands (up to kIslandMaxManifolds), manifolds sorted by (island, colour): a
 // workgroup solves a chunk of whole islands, every colour and pass, in one launch.
 struct island_sort
