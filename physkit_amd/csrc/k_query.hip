@@ -119,6 +119,23 @@ struct qslice
     }
 };
 
+// Whether a walk from the root reaches a leaf: the ray enters every box above it. A leaf that the ray
+// meets lies below such boxes, unless its box is not finite or flat (a body whose pose is NaN meets
+// every ray; a ray in a flat box' plane, parallel to it, is decided by the sign of a zero):
+// the boxes above leave such a leaf out or are decided otherwise, so it takes a climb.
+__device__ __forceinline__ bool reached(const lbvh_dev &t, const qray &q, uint32_t node)
+{
+    uint32_t p = t.parent[node];
+    for (uint32_t guard = 0; p != kNone && guard < 2 * t.n; ++guard)
+    {
+        const float4 lo = t.inode_lo[p], hi = t.inode_hi[p];
+        double td;
+        if (!ray_slab(q.o, q.inv, mk(lo.x, lo.y, lo.z), mk(hi.x, hi.y, hi.z), q.maxd, td)) return false;
+        p = t.parent[p];
+    }
+    return true;
+}
+
 // Calls leaf(body, distance) for every live leaf of the range (SLICED: of its slice s) that
 // the ray meets.
 template <bool SLICED, class Leaf>
@@ -162,7 +179,8 @@ __device__ __forceinline__ void walk_ray(const lbvh_dev &t, const bodies_dev &b,
                 const double *p = t.leaf_box + static_cast<size_t>(j) * 6;
                 double td;
                 if (b.is_static[body] != 2 &&
-                    ray_slab(q.o, q.inv, mk(p[0], p[1], p[2]), mk(p[3], p[4], p[5]), q.maxd, td))
+                    ray_slab(q.o, q.inv, mk(p[0], p[1], p[2]), mk(p[3], p[4], p[5]), q.maxd, td) &&
+                    (!SLICED || (p[0] < p[3] && p[1] < p[4] && p[2] < p[5]) || reached(t, q, node)))
                     leaf(body, td);
             }
         }

@@ -77,3 +77,45 @@ def test_either_side_of_the_lines(pk, extra, most):
         np.testing.assert_array_equal(f, boff[k:e + 1] - boff[k])
         np.testing.assert_array_equal(i, bids[boff[k]:boff[e]])
     g.close()
+
+
+@pytest.mark.parametrize("n", [33, 700, 5000])
+def test_bodies_without_a_finite_box(pk, n):
+    """Bodies whose pose is NaN or infinite and flat static bodies are hits of the same rays and boxes
+    whether a query's threads share its leaves or, with more queries, one thread walks the tree
+    from its root."""
+    s, rng = _scene(pk, n, 11)
+    bad = rng.choice(np.arange(1, n), 8, replace=False)
+    s["pos"][bad[0]] = np.nan
+    s["pos"][bad[1], 1] = np.nan
+    s["pos"][bad[2], 0] = np.inf
+    s["pos"][bad[3], 2] = -np.inf
+    s["quat"][bad[4]] = np.nan
+    # flat: a square in the plane y = 0 of the body
+    s["shape_offsets"] = np.append(s["shape_offsets"], s["shape_offsets"][-1] + 4).astype(np.uint32)
+    s["verts"] = np.concatenate([s["verts"], [[-1.0, 0, -1], [1, 0, -1], [1, 0, 1], [-1, 0, 1]]])
+    flat = bad[5:]
+    s["shape"][flat] = len(s["shape_offsets"]) - 2
+    s["is_static"][flat] = 1
+    s["quat"][flat] = [1.0, 0, 0, 0]
+    g = pk.GpuWorld(iterations=s["iterations"], flags=s["flags"])
+    g.load_scene(s)
+    o, d, m = _random_rays(rng, -2.0, 12.0, 2000, s["pos"][np.setdiff1d(np.arange(n), bad)])
+    o[:200] = s["pos"][flat[0]] + rng.normal(size=(200, 3)) * [3.0, 0.0, 3.0]
+    d[:200] = rng.normal(size=(200, 3))
+    d[:200, 1] = rng.choice([0.0, -0.0], 200)
+    m[:200] = np.inf
+    boxes = _boxes(rng, 1000, 2.0)
+    boxes[:10] = [-np.inf, -np.inf, -np.inf, np.inf, np.inf, np.inf]
+    boxes[10] = np.nan
+    rep, brep = 9, 9  # 18,000 rays and 9,000 boxes: past the lines
+    off, ids, dist = g.raycast(np.tile(o, (rep, 1)), np.tile(d, (rep, 1)), np.tile(m, rep))
+    boff, bids = g.query_aabb(np.tile(boxes, (brep, 1)))
+    f, i, t = g.raycast(o, d, m)
+    np.testing.assert_array_equal(f, off[:2001])
+    np.testing.assert_array_equal(i, ids[:f[-1]])
+    np.testing.assert_array_equal(t, dist[:f[-1]])
+    bf, bi = g.query_aabb(boxes)
+    np.testing.assert_array_equal(bf, boff[:1001])
+    np.testing.assert_array_equal(bi, bids[:bf[-1]])
+    g.close()
