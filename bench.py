@@ -140,7 +140,8 @@ def step_bytes(s, c, unique_vertices, scalar=8):
             + 10 * scalar * c["gjk_hits"] + c["contacts"] * (20 * scalar + 48))
 
 
-def stage_bytes(s, c, pairs, hits_frac, pos, iterations, mixed, tree_refits=0, integrate=True, steps=1):
+def stage_bytes(s, c, pairs, hits_frac, pos, iterations, mixed, tree_refits=0, integrate=True, steps=1,
+                one_kernel=False):
     """Compulsory HBM bytes of each stage's launches in one step, with the step's own
     counts (n bodies, N dynamic, M moved leaves, K candidate pairs, P pairs, H GJK hits,
     C manifold contacts, R solver rows; s_r = 4 for FP32 rows, else 8), averaged over
@@ -168,7 +169,9 @@ def stage_bytes(s, c, pairs, hits_frac, pos, iterations, mixed, tree_refits=0, i
                         (the manifold update rewrites the listed pairs), and a culled
                         pair writes no status byte (-1; the listed pairs' share of P is
                         a fraction of a percent and is not subtracted)
-      epa               algorithmic_bytes()
+      epa               algorithmic_bytes(); with one_kernel (short pair lists: k_gjk_epa_wave runs
+                        GJK and EPA) nothing, and gjk both stages' bytes without the
+                        simplex of each hit handed from one to the other (2 x 17 x 8)
       manifold          with per-body cull records, 28 L + 208 C + 192 H over the L pairs
                         GJK ran on (and the few culled pairs that had contacts): key,
                         source, status, previous count and slot, new count, slot and
@@ -202,9 +205,14 @@ def stage_bytes(s, c, pairs, hits_frac, pos, iterations, mixed, tree_refits=0, i
         "manifold": ("k_manifold" if fused else "k_manifold_live, k_manifold",
                      (0 if fused else 8 * P) + 28 * c["gjk_listed"] + 208 * C + 192 * H),
         "solver": ("contact solver stage", 496 * R),
-        "solve_iterations": ("k_solve_chunks" + ("<true> (FP32 rows)" if mixed else "<false>"), R * (38 * sr + 96)),
+        "solve_iterations": ("k_solve_chunks" + (" (FP32 rows)" if mixed else "") + ", with long islands k_solve_islands or k_solve",
+                             R * (38 * sr + 96)),
         "integrate_pos": ("k_integrate_pos", (n + 448 * nd) / steps),
     }
+    if one_kernel:
+        name, b = out["gjk"]
+        out["gjk"] = (name.replace("k_gjk)", "k_gjk_epa_wave)"), b + out["epa"][1] - 2 * 17 * 8 * H)
+        out["epa"] = ("none (k_gjk_epa_wave; larger-store reruns)", 0)
     if not integrate:
         out["integrate_vel"] = ("k_fill_u32 (moved flags cleared; integration off)", n)
         out["integrate_pos"] = ("none (integration off)", 0)
@@ -222,7 +230,7 @@ def roofline_of(stage_ms, steps, models):
         t = (rest if k == "solver" else ms.get(k, 0.0)) / steps
         gbs = b / (t / 1e3) / 1e9 if t > 0 else 0.0
         table[k] = {"kernel": name if k != "solver" else "contact solver stage without its iterations "
-                    "(k_row_flags, colouring, islands, k_setup, k_writeback)",
+                    "(k_row_flags, islands; with long islands colouring, k_setup, k_writeback)",
                     "avg_launch_ms": round(t, 4), "algorithmic_bytes": float(b), "achieved_GBs": round(gbs, 2),
                     "frac": round(gbs / HBM_PEAK_GBS, 5)}
     dom = max(table, key=lambda k: table[k]["avg_launch_ms"])
@@ -315,8 +323,9 @@ def timed_run(pk, s, flags, warmup, steps, autotune=True, fixed=None, tree_refit
     g.load_scene(s)
     if len(s["first_body"]) > 2:
         g.set_worlds(s["first_body"])
+    default = g.tuning()
     if tuning is None:
-        tuning = g.tuning()
+        tuning = default
     g.set_tuning(tuning["gjk_lanes"], tuning["epa_block"], tuning["epa_lds_max"], tree_refits)
     tuning = dict(tuning, tree_refits=tree_refits)
     for _ in range(warmup):
@@ -333,6 +342,9 @@ def timed_run(pk, s, flags, warmup, steps, autotune=True, fixed=None, tree_refit
     hits_total = c["gjk_hits_total"] - c0["gjk_hits_total"]
     out = {"wall": wall, "stage": stage, "pairs_total": pairs_total, "hits_total": hits_total,
            "counters": g.counters(), "pairs": g.pairs(), "pos": g.bodies()["pos"], "tuning": tuning}
+    # GJK and EPA in one kernel: the default shapes and at most 8,192 pairs expected (pkg_tuning)
+    out["one_kernel"] = (all(tuning[k] == default[k] for k in ("gjk_lanes", "epa_block", "epa_lds_max"))
+                         and 1.25 * c["gjk_fp64"] <= 8192)
     g.close()
     return out
 
@@ -564,8 +576,8 @@ def main():
                     help="keep the default launch shapes instead of those pkg_autotune picks on a copy "
                          "of the world")
     ap.add_argument("--tuning", default=None, metavar="LANES,BLOCK,LDS_MAX",
-                    help="fixed launch shapes (GJK lanes per pair, EPA workgroup size, LDS-store "
-                         "threshold) instead of pkg_autotune's, e.g. to profile the shapes a bench "
+                    help="fixed launch shapes (GJK lanes per pair, EPA workgroup size, most hits "
+                         "that get a wavefront each) instead of pkg_autotune's, e.g. to profile the shapes a bench "
                          "line reports")
     ap.add_argument("--tree-refits", type=int, default=TREE_REFITS, metavar="N",
                     help="steps between full LBVH builds that refit the last hierarchy instead "
@@ -606,7 +618,7 @@ def main():
     hits_frac = c["gjk_hits"] / max(c["pairs"], 1)
     models = stage_bytes(s, c, pairs, hits_frac, r["pos"], s["iterations"], mixed or prec == "fp32-solve",
                          args.tree_refits, integrate=(int(s["flags"]) & pk.FLAG_NO_INTEGRATE) == 0,
-                         steps=args.steps)
+                         steps=args.steps, one_kernel=r["one_kernel"])
     dom, table = roofline_of(stage, args.steps, models)
     d = table[dom]
     roof = {"bound": "hbm", "stage": dom, "kernel": d["kernel"], "achieved": d["achieved_GBs"],
@@ -633,7 +645,7 @@ def main():
                    "colliding_pairs_per_s": round(r["hits_total"] / wall, 1),
                    "stage_ms_per_step": {k: round(v / args.steps, 4) for k, v in stage.items()},
                    "stage_roofline": table,
-                   "launch_shapes": r["tuning"],
+                   "launch_shapes": dict(r["tuning"], gjk_and_epa_in_one_kernel=r["one_kernel"]),
                    "step_algorithmic_bytes": step_b,
                    "step_hbm_frac": round(step_b / (wall / args.steps) / (HBM_PEAK_GBS * 1e9), 5),
                    "worlds": len(s["first_body"]) - 1,

@@ -329,7 +329,8 @@ typedef struct pkg_tuning
  * keeps the fastest of each: GJK lanes on the GJK stage, the EPA block size with every
  * batch per thread, then epa_lds_max with the step's fastest block size; and, over the steps
  * with at most 8,192 pairs for GJK, whichever is faster of the one kernel and the
- * fastest separate ones. pkg_upload_bodies returns gjk_lanes and this last choice to the
+ * fastest separate ones (the one kernel on every step: the shapes are left at the defaults, so
+ * that pkg_set_tuning with them gives another world the one kernel as well). pkg_upload_bodies returns gjk_lanes and this last choice to the
  * defaults. out (optional) receives the choice and the
  * mean times measured. */
 pkg_status pkg_autotune(pkg_ctx *ctx, double dt, int steps, pkg_tuning *out);

@@ -257,6 +257,7 @@ struct pkg_ctx
         // steps with lists short enough for it: the fused kernel, and the fastest GJK and
         // EPA shapes as separate kernels
         double fused = 0, separate = 0;
+        int short_steps = 0;
     } *trials = nullptr;
     dbuf<double> simplex, info;
     dbuf<uint8_t> status;
@@ -963,6 +964,7 @@ void pkg_ctx::step_once(double dt, hipEvent_t *ev, bool defer_pos)
             if (is_short)
             {
                 trials->fused += fused_ms;
+                ++trials->short_steps;
                 trials->separate += *std::min_element(gjk_ms, gjk_ms + 4) + *std::min_element(ms, ms + 3);
             }
         }
@@ -2032,6 +2034,15 @@ pkg_status pkg_autotune(pkg_ctx *ctx, double dt, int steps, pkg_tuning *out)
             tu.epa_block = blocks[argmin(tr.epa_block, 3)];
             tu.epa_lds_max = lds_max[argmin(tr.epa_lds, 3)];
             tu.fuse = tr.fused <= tr.separate; // no short list seen: as by default
+            if (tu.fuse && tr.short_steps == steps)
+            {
+                // the shapes were not needed: the defaults, which pkg_set_tuning on another
+                // world takes for the one kernel too
+                const tuning d{};
+                tu.gjk_group = ctx->default_gjk_group();
+                tu.epa_block = d.epa_block;
+                tu.epa_lds_max = d.epa_lds_max;
+            }
             for (int c = 0; c < 4; ++c) res.gjk_ms[c] = static_cast<float>(tr.gjk[c] / steps);
             for (int c = 0; c < 3; ++c)
             {

@@ -110,3 +110,17 @@ def test_stage_bytes_manifold_forms():
     out10 = bench.stage_bytes(s, c10, every, 0.1, s["pos"], 10, False)
     assert out10["manifold"][1] == 28 * 3 + 208 * 2 + 192 * 1
     assert out10["gjk"][1] == bench.algorithmic_bytes("gjk", s, every, 0.1, s["pos"]) + 6 * 10
+
+
+def test_stage_bytes_one_kernel():
+    """GJK and EPA in one kernel: its row has both stages' bytes but the simplices handed over."""
+    b = _box(0.5)
+    s = _scene([b], [0, 0], [[0, 0, 0], [0.9, 0, 0]])
+    s["n_static"] = 0
+    pairs = np.array([(0 << 32) | 1], np.uint64)
+    c = _counters(pairs=1, gjk_listed=1, gjk_hits=1)
+    two = bench.stage_bytes(s, c, pairs, 1.0, s["pos"], 10, False)
+    one = bench.stage_bytes(s, c, pairs, 1.0, s["pos"], 10, False, one_kernel=True)
+    assert one["gjk"][1] == two["gjk"][1] + two["epa"][1] - 2 * 17 * 8
+    assert one["epa"][1] == 0 and "k_gjk_epa_wave" in one["gjk"][0]
+    assert all(one[k] == two[k] for k in two if k not in ("gjk", "epa"))

@@ -194,6 +194,11 @@ def test_short_lists_keep_the_fused_kernel(pk):
         print(f"[tuning] {name}: EPA stage {ms:.4f} ms, separate kernels {separate:.4f} ms", flush=True)
         assert ms < 0.5 * separate, name
         _same(name, got, want)
-    ms, _ = epa_ms(lambda g: g.autotune(s["dt"], 8))
-    print(f"[tuning] autotune: EPA stage {ms:.4f} ms", flush=True)
+    found = {}
+    ms, _ = epa_ms(lambda g: found.update(g.autotune(s["dt"], 8)))
+    print(f"[tuning] autotune: EPA stage {ms:.4f} ms, {found}", flush=True)
     assert ms < 0.5 * separate
+    # what it returned, set on another world, keeps the kernel there
+    ms, got = epa_ms(lambda g: g.set_tuning(found["gjk_lanes"], found["epa_block"], found["epa_lds_max"]))
+    assert ms < 0.5 * separate
+    _same("shapes of autotune", got, want)
