@@ -887,7 +887,8 @@ void pkg_ctx::step_once(double dt, hipEvent_t *ev, bool defer_pos)
         {
             if (!novf) return;
             ovf2_list.reserve(novf);
-            launch_epa_wave(keys[nxt].p, ovf_list.p, novf, b, s, has_uv, true, g, ovf2_list.p, counters.p + C_EPA_OVF2, st);
+            launch_epa_wave(keys[nxt].p, ovf_list.p, novf, b, s, has_uv, true, g, ovf2_list.p, counters.p + C_EPA_OVF2,
+                            tune.wave_launch, st);
             const uint32_t n2 = static_cast<uint32_t>(read_counter(C_EPA_OVF2));
             if (!n2) return;
             big_pool.reserve(static_cast<size_t>(n2) * epa_big_bytes());
@@ -1302,6 +1303,9 @@ pkg_status pkg_create(pkg_ctx **out, const pkg_config *cfg)
         c->counters.reserve(C_NCOUNTERS);
         if (const char *e = std::getenv("PKG_PAIR_REGION_MIN_LEAVES"))
             c->region_min_leaves = static_cast<uint32_t>(std::strtoul(e, nullptr, 10));
+        // wavefronts a launch in place of kWaveLaunch (tests split short lists with it)
+        if (const char *e = std::getenv("PKG_WAVE_LAUNCH"))
+            c->tune.wave_launch = std::clamp<uint32_t>(static_cast<uint32_t>(std::strtoul(e, nullptr, 10)), 1, kWaveLaunch);
         c->scene.reserve(12);
     }
     catch (const pk_error &e)
@@ -2288,7 +2292,7 @@ pkg_status pkg_gjk_epa_batch(pkg_ctx *ctx, uint32_t n, const int32_t *kind_a, co
         sp.verts = dv.p;
         sp.uv_a = ua.p;
         sp.uv_b = ub.p;
-        launch_gjk_epa_batch_dev(sp, n, n_verts, dout.p, dh.p, words.p, ovf.p, pool.p, 1, st);
+        launch_gjk_epa_batch_dev(sp, n, n_verts, dout.p, dh.p, words.p, ovf.p, pool.p, 1, ctx->tune.wave_launch, st);
         hip_check(hipGetLastError(), "batch launch");
         std::vector<double> o = download(dout, 10 * static_cast<size_t>(n), st);
         std::vector<int32_t> h = download(dh, n, st);
@@ -2338,7 +2342,7 @@ pkg_status pkg_gjk_epa_batch_device(pkg_ctx *ctx, uint32_t n, const int32_t *kin
         sp.verts = verts;
         sp.uv_a = nullptr; // no UV-sphere tags: full support scans, the same results
         sp.uv_b = nullptr;
-        launch_gjk_epa_batch_dev(sp, n, n_verts, out, hit, sc->words, sc->ovf_list, sc->stores, kNoAllocStores,
+        launch_gjk_epa_batch_dev(sp, n, n_verts, out, hit, sc->words, sc->ovf_list, sc->stores, kNoAllocStores, ctx->tune.wave_launch,
                                  ctx->st);
         hip_check(hipGetLastError(), "batch launch");
         // the counters into the ctx's pinned words (allocated by pkg_create)

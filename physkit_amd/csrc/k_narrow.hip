@@ -720,11 +720,12 @@ __global__ void k_batch_dev_big(shape_pair_dev sp, double *out, int32_t *hit, ui
 size_t epa_big_bytes() { return sizeof(epa_store_big); }
 
 void launch_gjk_epa_batch_dev(const shape_pair_dev &sp, uint32_t n, uint32_t n_verts, double *out, int32_t *hit,
-                              uint32_t *words, uint32_t *ovf_list, void *stores, uint32_t n_stores, hipStream_t st)
+                              uint32_t *words, uint32_t *ovf_list, void *stores, uint32_t n_stores, uint32_t per_launch,
+                              hipStream_t st)
 {
     k_batch_dev_clear<<<1, 64, 0, st>>>(words);
     if (!n) return;
-    launch_batch_wave(sp, n, n_verts, out, hit, words, ovf_list, st);
+    launch_batch_wave(sp, n, n_verts, out, hit, words, ovf_list, per_launch, st);
     k_batch_dev_big<<<1, 64, 0, st>>>(sp, out, hit, words, ovf_list, static_cast<epa_store_big *>(stores), n_stores);
 }
 
@@ -782,7 +783,7 @@ void launch_epa(const uint64_t *keys, uint32_t n_hits, const bodies_dev &b, cons
     if (!n_hits) return;
     if (n_hits <= tu.epa_lds_max)
     {
-        launch_epa_wave(keys, nullptr, n_hits, b, s, uv, false, g, ovf_list, &counters[C_EPA_OVF], st);
+        launch_epa_wave(keys, nullptr, n_hits, b, s, uv, false, g, ovf_list, &counters[C_EPA_OVF], tu.wave_launch, st);
         return;
     }
     auto go = [&](auto block)

@@ -85,12 +85,13 @@ __global__ void __launch_bounds__(kWave)
 // hull hits 1.56 -> 1.35 ms); with UV spheres they spill (56,000 mixed hits 0.44 -> 0.49).
 template <bool UV, int K>
 __global__ void __launch_bounds__(kWave, K == kStepSlots && !UV ? 4 : 1)
-    k_epa_wave(const uint64_t *keys, const uint32_t *in_list, uint32_t n, bodies_dev b, shapes_dev s, gjk_out_dev g,
-               uint32_t *ovf_list, unsigned long long *ovf_count)
+    k_epa_wave(const uint64_t *keys, const uint32_t *in_list, uint32_t first, uint32_t n, bodies_dev b, shapes_dev s,
+               gjk_out_dev g, uint32_t *ovf_list, unsigned long long *ovf_count)
 {
     __shared__ wave::store<K> st;
-    if (blockIdx.x >= n) return;
-    const uint32_t h = in_list ? wave::first32(in_list[blockIdx.x]) : blockIdx.x;
+    const uint32_t i = first + blockIdx.x;
+    if (i >= n) return;
+    const uint32_t h = in_list ? wave::first32(in_list[i]) : i;
     const uint32_t p = wave::first32(g.hit_list[h]);
     const wave::shape w = pair_side<UV>(b, s, keys[p]);
     simplex x;
@@ -109,7 +110,7 @@ __global__ void __launch_bounds__(kWave, K == kStepSlots && !UV ? 4 : 1)
 template <bool UV>
 __global__ void __launch_bounds__(kWave)
     k_batch_wave(shape_pair_dev sp, uint32_t n, uint32_t n_verts, double *out, int32_t *hit, uint32_t *words,
-                 uint32_t *ovf_list)
+                 uint32_t *ovf_list, uint32_t first)
 {
     __shared__ wave::store<kBatchSlots> st;
     const uint32_t i = blockIdx.x;
@@ -141,7 +142,14 @@ __global__ void __launch_bounds__(kWave)
     if (r == 1)
         for (int c = 0; c < 10; ++c) out[10 * static_cast<size_t>(i) + c] = o[c];
     hit[i] = r == 1 ? 1 : (r == 0 ? 2 : 3);
-    if (r == 3) ovf_list[atomicAdd(&words[1], 1u)] = i;
+    if (r == 3) ovf_list[atomicAdd(&words[1], 1u)] = first + i;
+}
+
+// one workgroup of a wavefront per item, at most per_launch of them in a launch
+template <class Launch> void in_parts(uint32_t n, uint32_t per_launch, Launch &&launch)
+{
+    for (uint64_t first = 0; first < n; first += per_launch)
+        launch(static_cast<uint32_t>(first), static_cast<uint32_t>(std::min<uint64_t>(per_launch, n - first)));
 }
 } // namespace
 
@@ -158,16 +166,19 @@ void launch_gjk_epa_wave(const uint64_t *keys, const uint32_t *list, int list_sl
 
 void launch_epa_wave(const uint64_t *keys, const uint32_t *in_list, uint32_t n, const bodies_dev &b, const shapes_dev &s,
                      bool uv, bool rerun, const gjk_out_dev &g, uint32_t *ovf_list, unsigned long long *ovf_count,
-                     hipStream_t st)
+                     uint32_t per_launch, hipStream_t st)
 {
-    if (!n) return;
     auto go = [&](auto slots)
     {
         constexpr int K = decltype(slots)::value;
-        if (uv)
-            k_epa_wave<true, K><<<n, kWave, 0, st>>>(keys, in_list, n, b, s, g, ovf_list, ovf_count);
-        else
-            k_epa_wave<false, K><<<n, kWave, 0, st>>>(keys, in_list, n, b, s, g, ovf_list, ovf_count);
+        in_parts(n, per_launch,
+                 [&](uint32_t first, uint32_t wgs)
+                 {
+                     if (uv)
+                         k_epa_wave<true, K><<<wgs, kWave, 0, st>>>(keys, in_list, first, n, b, s, g, ovf_list, ovf_count);
+                     else
+                         k_epa_wave<false, K><<<wgs, kWave, 0, st>>>(keys, in_list, first, n, b, s, g, ovf_list, ovf_count);
+                 });
     };
     if (rerun)
         go(std::integral_constant<int, kBatchSlots>{});
@@ -176,13 +187,24 @@ void launch_epa_wave(const uint64_t *keys, const uint32_t *in_list, uint32_t n, 
 }
 
 void launch_batch_wave(const shape_pair_dev &sp, uint32_t n, uint32_t n_verts, double *out, int32_t *hit, uint32_t *words,
-                       uint32_t *ovf_list, hipStream_t st)
+                       uint32_t *ovf_list, uint32_t per_launch, hipStream_t st)
 {
-    if (!n) return;
-    if (sp.uv_a)
-        k_batch_wave<true><<<n, kWave, 0, st>>>(sp, n, n_verts, out, hit, words, ovf_list);
-    else
-        k_batch_wave<false><<<n, kWave, 0, st>>>(sp, n, n_verts, out, hit, words, ovf_list);
+    in_parts(n, per_launch,
+             [&](uint32_t first, uint32_t wgs)
+             {
+                 shape_pair_dev part = sp; // entries first, first + 1, ...
+                 for (const int32_t **p : {&part.kind_a, &part.kind_b}) *p += first;
+                 for (const uint32_t **p : {&part.vbeg_a, &part.vend_a, &part.vbeg_b, &part.vend_b}) *p += first;
+                 for (const double **p : {&part.prm_a, &part.prm_b}) *p += 10 * static_cast<size_t>(first);
+                 if (sp.uv_a)
+                 {
+                     part.uv_a += first;
+                     part.uv_b += first;
+                 }
+                 auto kernel = sp.uv_a ? k_batch_wave<true> : k_batch_wave<false>;
+                 kernel<<<wgs, kWave, 0, st>>>(part, wgs, n_verts, out + 10 * static_cast<size_t>(first), hit + first, words,
+                                               ovf_list, first);
+             });
 }
 
 } // namespace pk

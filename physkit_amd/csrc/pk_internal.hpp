@@ -312,6 +312,10 @@ struct cull_manifold_out
 void launch_gjk(const uint64_t *keys, uint32_t n_pairs, const bodies_dev &b, const shapes_dev &s, bool uv, int group,
                 gjk_out_dev &g, uint32_t *list, double *cull_rec, const gjk32_in &f32, const gjk_wave_in &wv,
                 const cull_manifold_out &mo, unsigned long long *counters, hipStream_t st);
+// Wavefronts that one launch gives an item each: a grid counts its work-items in 32 bits, so
+// 67,108,863 wavefronts are the most. Longer lists take several launches.
+constexpr uint32_t kWaveLaunch = 1u << 25;
+static_assert(kWaveLaunch * 64ull <= 0xFFFFFFFFull);
 // Launch shapes the autotuner picks (pkg_autotune); none changes a result.
 struct tuning
 {
@@ -320,6 +324,7 @@ struct tuning
     uint32_t epa_lds_max = 0xFFFFFFFFu; // batches of at most this many GJK hits run one EPA solve per
                                         // wavefront (k_epa_wave); larger ones one per thread (k_epa)
     uint32_t tree_refits = 7;    // steps that refit the last LBVH hierarchy between full builds
+    uint32_t wave_launch = kWaveLaunch;
     bool fuse = true; // lists expected to be short run GJK and EPA in one kernel (kWavePairs)
 };
 void launch_epa(const uint64_t *keys, uint32_t n_hits, const bodies_dev &b, const shapes_dev &s, bool uv,
@@ -328,7 +333,7 @@ void launch_epa(const uint64_t *keys, uint32_t n_hits, const bodies_dev &b, cons
 // rerun of overflows; its own overflows are listed in ovf_list (count at *ovf_count)
 void launch_epa_wave(const uint64_t *keys, const uint32_t *in_list, uint32_t n, const bodies_dev &b, const shapes_dev &s,
                      bool uv, bool rerun, const gjk_out_dev &g, uint32_t *ovf_list, unsigned long long *ovf_count,
-                     hipStream_t st);
+                     uint32_t per_launch, hipStream_t st);
 size_t epa_big_bytes();
 void launch_epa_big(const uint64_t *keys, const uint32_t *ovf_list, uint32_t n_ovf,
                     const bodies_dev &b, const shapes_dev &s, gjk_out_dev &g, void *pool,
@@ -358,13 +363,13 @@ struct shape_pair_dev
 };
 // one wavefront per pair; overflows of its store are listed (words[1]) in ovf_list
 void launch_batch_wave(const shape_pair_dev &sp, uint32_t n, uint32_t n_verts, double *out, int32_t *hit, uint32_t *words,
-                       uint32_t *ovf_list, hipStream_t st);
+                       uint32_t *ovf_list, uint32_t per_launch, hipStream_t st);
 // The batch over device arrays: words (4 x u32:
 // invalid pairs, pairs listed for the large store, pairs that overflowed it too; cleared
 // by the first launch), ovf_list (n entries) and n_stores large EPA stores. Invalid pairs
 // get hit = -1. uv tags may be null.
 void launch_gjk_epa_batch_dev(const shape_pair_dev &sp, uint32_t n, uint32_t n_verts, double *out, int32_t *hit,
-                              uint32_t *words, uint32_t *ovf_list, void *stores, uint32_t n_stores, hipStream_t st);
+                              uint32_t *words, uint32_t *ovf_list, void *stores, uint32_t n_stores, uint32_t per_launch, hipStream_t st);
 
 // ---------------- k_solver.hip ----------------
 struct rows_dev

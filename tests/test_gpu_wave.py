@@ -132,3 +132,37 @@ def test_list_that_grows_at_once(pk):
         _assert_same("dense", i, a, b)
     print(f"[wave] dense step: default {ms[0]:.3f} ms, separate kernels {ms[1]:.3f} ms", flush=True)
     assert ms[0] <= 2.0 * ms[1]
+
+
+def test_lists_longer_than_a_launch(pk, monkeypatch):
+    """Lists of more wavefronts than one launch can count (2^25) go in several: with 97 a launch (read
+    from PKG_WAVE_LAUNCH when a context is created) the batch and a step's EPA, reruns of
+    overflows among them, give what single launches give."""
+    rng = np.random.default_rng(4714)
+    pairs = [((2, np.concatenate([rng.normal(size=3) * 0.1, _quat(rng)]), _hull(rng, int(rng.integers(1, 40)))),
+              (2, np.concatenate([rng.normal(size=3) * 0.3, _quat(rng)]), _hull(rng, int(rng.integers(1, 40)))))
+             for _ in range(400)]
+    sph = pk.mesh.sphere(0.5, 16, 32).vertices
+    n = 400  # deep pairs of spheres, each far from the others: all hit, some past 192 faces
+    u = rng.normal(size=(n // 2, 3))
+    u *= rng.uniform(0.05, 0.6, (n // 2, 1)) / np.linalg.norm(u, axis=1, keepdims=True)
+    a = np.stack([5.0 * (np.arange(n // 2) % 20), np.zeros(n // 2), 5.0 * (np.arange(n // 2) // 20)], 1)
+    s = {"shape_offsets": np.array([0, len(sph)], np.uint32), "verts": sph, "is_static": np.zeros(n, np.uint8),
+         "shape": np.zeros(n, np.uint32), "pos": np.stack([a, a + u], 1).reshape(n, 3), "vel": np.zeros((n, 3)),
+         "angvel": np.zeros((n, 3)), "quat": np.array([_quat(rng) for _ in range(n)]), "mass": np.ones(n),
+         "inertia": np.tile(np.eye(3).reshape(9) * 0.1, (n, 1)), "restitution": np.full(n, 0.5), "friction": np.full(n, 0.5)}
+    got = []
+    for per in (None, "97", "1"):
+        if per:
+            monkeypatch.setenv("PKG_WAVE_LAUNCH", per)
+        g = pk.GpuWorld(iterations=4, flags=pk.FLAG_ALL_MOVED | pk.FLAG_NO_SOLVER | pk.FLAG_NO_INTEGRATE)
+        g.load_scene(s)
+        g.set_tuning(2, 64, 1 << 20)
+        g.step(1 / 60)
+        c = g.counters()
+        assert c["gjk_hits"] == n // 2 and c["epa_overflow"] > 0
+        got.append((*g.manifolds(), *g.gjk_epa_batch([p[0] for p in pairs], [p[1] for p in pairs])))
+        g.close()
+    for other in got[1:]:
+        for i, (x, y) in enumerate(zip(got[0], other)):
+            _assert_same("launches", i, y, x)
