@@ -3,7 +3,7 @@
 //   integrate_vel + leaf update -> pairs -> narrowphase -> contact setup/solve ->
 //   integrate_pos.
 // Host synchronisation points (counts that size the next launch): candidate count,
-// pair count, GJK hit count, EPA overflow count, solver rows, colour rounds.
+// pair count, GJK hit count, EPA overflow count, solver rows and island lengths, colour rounds.
 #include "physkit_amd.h"
 #include "pk_access.hpp"
 #include "pk_copy.hpp"

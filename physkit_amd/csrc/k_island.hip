@@ -10,8 +10,11 @@
 // takes two lanes, one for each body: a lane holds its body's inverse mass and inertia and
 // lever arms, computes its half of every J.v and applies its half of every impulse, and the
 // halves meet through a DPP exchange with the neighbour lane, in the order of operations of
-// the sequential solve (bit for bit). Rows never go to memory: a lane builds them in
-// registers from the manifold and keeps them across the passes; velocities are in LDS.
+// the sequential solve (bit for bit). A lane builds its manifold's rows from the manifold and keeps
+// them across the passes; velocities are in LDS. FP32 rows fit its registers (171). FP64 rows
+// of four contacts do not: both FP64 forms use all 256 that 512 threads leave a lane and
+// spill 63 and 64 more to private memory (168 and 164 bytes a lane), 19 loads of which lie
+// in the loop over passes and colours.
 // Colours come from the same rounds as the global colouring (k_solver.hip), on LDS claims.
 //
 // Measured, solver stage per step, against global colouring rounds (three launches each),

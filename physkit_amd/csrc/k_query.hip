@@ -19,7 +19,11 @@ constexpr int kBlock = 256;
 // Up to this many rays or boxes kSlices threads share one; beyond, the chip is full without and
 // the slices' first steps only add work. Whole calls over 32,768 bodies with 1, 16 and 32
 // slices: 1,024 rays 1.23, 0.97 and 0.81 ms, 16,384 rays 1.51, 1.26 and 1.19, 65,536 rays
-// 2.09, 2.27 and 2.66; 4,096 boxes 1.53, 1.31 and 1.22, 16,384 boxes 1.74, 1.95 and 1.89.
+// 2.09, 2.27 and 2.66; 4,096 boxes 1.53, 1.31 and 1.22, 16,384 boxes 1.74, 1.95 and 1.89. The
+// bodies do not move the line: with one thread a query and radix sorts, and so, 16,384 rays over 64
+// bodies took 0.71 and 0.38 ms, over 1,024 1.46 and 0.65, over 262,144 3.32 and 1.70; 16 rays
+// 0.44 and 0.28, 0.68 and 0.36, 1.28 and 0.80; 8,192 boxes 0.50 and 0.29, 1.62 and 0.61, 2.42
+// and 1.75.
 constexpr uint32_t kSliceRays = 16384;
 constexpr uint32_t kSliceBoxes = 8192;
 constexpr uint32_t kSlices = 32;

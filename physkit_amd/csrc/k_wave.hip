@@ -81,8 +81,9 @@ __global__ void __launch_bounds__(kWave)
 
 // EPA of hits in_list[0..n) (0..n-1 when null), one wavefront each: 0.12 ms on 8,400 hull hits
 // (one thread each 0.45), 0.44 on 56,000 mixed hits (0.96), 0.13 on 17,880 box hits (0.36) and
-// 1.35 on 143,000 hull hits (2.07). Four wavefronts a SIMD where 128 registers do (143,000
-// hull hits 1.56 -> 1.35 ms); with UV spheres they spill (56,000 mixed hits 0.44 -> 0.49).
+// 1.35 on 143,000 hull hits (2.07). Four wavefronts a SIMD without UV spheres, though 13
+// registers then spill (143,000 hull hits 1.56 -> 1.35 ms); with them too many do (56,000 mixed
+// hits 0.44 -> 0.49).
 template <bool UV, int K>
 __global__ void __launch_bounds__(kWave, K == kStepSlots && !UV ? 4 : 1)
     k_epa_wave(const uint64_t *keys, const uint32_t *in_list, uint32_t first, uint32_t n, bodies_dev b, shapes_dev s,

@@ -439,8 +439,8 @@ void launch_island_group(const uint32_t *list, uint32_t nl, const uint32_t *cnt,
 // solve, whose longer islands keep the row arithmetic of launch_solve_islands, and whose islands of
 // more than kIslandMaxColours colours that of launch_solve_colour32). isl null: the list (at most
 // kChunkTwoLanes) is one chunk. root: each position's island root. Two lanes per manifold up to 256 manifolds: 512
-// threads, the most whose FP64 rows of four contacts fit the 256 registers a thread then has;
-// one lane, with its lever arms in LDS, up to 512.
+// threads, the most that leave a thread 256 registers, which FP64 rows of four contacts fill
+// and pass by 63; one lane, with its lever arms in LDS, up to 512.
 constexpr int kChunkTwoLanes = 256, kChunkMax = 512, kChunkMax32 = 256;
 constexpr uint32_t kChunkFill = 32; // manifolds a chunk takes before another workgroup is opened
 void launch_solve_chunks(const uint64_t *keys, const uint32_t *ord, const uint32_t *isl, const uint32_t *root, uint32_t nl,

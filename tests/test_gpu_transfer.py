@@ -1,5 +1,6 @@
 """Body state between the caller's arrays and the device, where its route changes: up to 256
-KiB the kernels use pinned memory directly, above it goes through 16 MiB halves. Downloads
+KiB the kernels use pinned memory directly, up to 16 MiB it goes through device memory in one
+piece, above in 16 MiB halves. Downloads
 return the uploaded state bit for bit, any subset of the arrays, and set_state reaches the
 named bodies alone."""
 import ctypes as C

@@ -1,8 +1,8 @@
 """Launch shapes (pkg_set_tuning / pkg_autotune) change timings, never results: every
-combination of GJK lanes per pair, EPA workgroup size and LDS threshold steps the same
-world to bit-identical bodies, pairs and manifolds, and pkg_autotune (which reruns the
-GJK and EPA stages of each step it takes with every candidate) advances the world
-exactly as plain steps would."""
+combination of GJK lanes per pair, EPA workgroup size and epa_lds_max (a thread or a
+wavefront per EPA solve) steps the same world to bit-identical bodies, pairs and manifolds,
+and pkg_autotune (which reruns the GJK and EPA stages of each step it takes with every
+candidate) advances the world exactly as plain steps would."""
 import itertools
 
 import numpy as np
@@ -125,8 +125,8 @@ def test_set_tuning_rejects_unknown_shapes(pk):
 
 def test_epa_tiers_and_overflows_bitexact(pk, oracle):
     """Deeply overlapping 16x32 UV spheres (up to 64 expansions and 319 faces per EPA
-    solve, more than the 192 faces of the first tier's store): every first EPA tier
-    (the private store at each workgroup size, the 896-face LDS store), with its
+    solve, more than the 192 faces of the first tier's store): either first EPA tier
+    (the private store at each workgroup size, a wavefront's registers), with its
     overflows rerun in the larger stores, reaches the oracle's manifolds bit for bit."""
     from test_gpu_parity import _compare_world
     rng = np.random.default_rng(29)
