@@ -287,7 +287,8 @@ pkg_status pkg_query_aabb(pkg_ctx *ctx, uint32_t n_boxes, const double *boxes, c
 
 /* pkg_step with per-stage device time, measured with HIP events on the ctx stream.
  * Stages: 0 integrate_vel + leaf update, 1 LBVH build, 2 pair-set update, 3 GJK
- * stage (cull, FP32 pass, GJK kernel), 4 EPA kernel(s), 5 manifold update kernel,
+ * stage (cull, FP32 pass, GJK kernel; on short lists the kernel that runs GJK and EPA),
+ * 4 EPA kernel(s) of its own, 5 manifold update kernel,
  * 6 contact solver (rows, colouring, islands, iterations, impulse write-back),
  * 7 integrate_pos, 8 the solver's iteration kernels alone (part of stage 6).
  * stage_ms[i] is the sum over the nsteps steps (up to 9 entries). */
